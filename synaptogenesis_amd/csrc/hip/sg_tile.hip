@@ -5,38 +5,76 @@
 
 namespace sg {
 
-template <int WAVES, int CHUNK>
-static hipError_t launch_tile_base_t(const sg_conn &c, hipStream_t st) {
-    dim3 g((c.num_dest + 63) / 64), b(64 * WAVES);
-#define SG_TB(T)                                                             \
-    switch (c.out_type) {                                                    \
-        case SG_OUT_BIT:                                                     \
-            hipLaunchKernelGGL((tile_base_kernel<T, SG_OUT_BIT, WAVES,       \
-                                CHUNK>), g, b, 0, st, c); break;             \
-        case SG_OUT_INT:                                                     \
-            hipLaunchKernelGGL((tile_base_kernel<T, SG_OUT_INT, WAVES,       \
-                                CHUNK>), g, b, 0, st, c); break;             \
-        default:                                                             \
-            hipLaunchKernelGGL((tile_base_kernel<T, SG_OUT_FLOAT, WAVES,     \
-                                CHUNK>), g, b, 0, st, c);                    \
+template <int TYPE, int D, int WAVES>
+static void launch_tile_type(const sg_conn &c, hipStream_t st) {
+    dim3 g((c.num_dest + D - 1) / D), b(64 * WAVES);
+    switch (c.out_type) {
+        case SG_OUT_BIT:
+            hipLaunchKernelGGL((tile_base_kernel<TYPE, SG_OUT_BIT, D, WAVES>),
+                               g, b, 0, st, c);
+            break;
+        case SG_OUT_INT:
+            hipLaunchKernelGGL((tile_base_kernel<TYPE, SG_OUT_INT, D, WAVES>),
+                               g, b, 0, st, c);
+            break;
+        default:
+            hipLaunchKernelGGL((tile_base_kernel<TYPE, SG_OUT_FLOAT, D,
+                                WAVES>), g, b, 0, st, c);
     }
-    switch (c.type) {
-        case SG_FULLY_CONNECTED: SG_TB(SG_FULLY_CONNECTED); break;
-        case SG_SUBSET: SG_TB(SG_SUBSET); break;
-        case SG_CONVERGENT: SG_TB(SG_CONVERGENT); break;
-        case SG_DIVERGENT: SG_TB(SG_DIVERGENT); break;
-        case SG_SPARSE: SG_TB(SG_SPARSE); break;
-        default: return hipErrorInvalidValue;
+}
+
+template <int TYPE>
+static void launch_lane_type(const sg_conn &c, hipStream_t st) {
+    dim3 g((c.num_dest + 63) / 64), b(64);
+    switch (c.out_type) {
+        case SG_OUT_BIT:
+            hipLaunchKernelGGL((lane_base_kernel<TYPE, SG_OUT_BIT>), g, b, 0,
+                               st, c);
+            break;
+        case SG_OUT_INT:
+            hipLaunchKernelGGL((lane_base_kernel<TYPE, SG_OUT_INT>), g, b, 0,
+                               st, c);
+            break;
+        default:
+            hipLaunchKernelGGL((lane_base_kernel<TYPE, SG_OUT_FLOAT>), g, b,
+                               0, st, c);
     }
-#undef SG_TB
+}
+
+// Which form of the base activator (all three give the same bits), from one
+// sweep of sizes:
+// * lanes alone once the layer's own wavefronts fill the GPU and the visits'
+//   sources have to be walked: convergent 5 x 5 on 256 x 256 (1024 tiles)
+//   6.1 us against 9.8, 15 x 15 on 360 x 360 (2025 tiles) 37.5 against 45
+//   (on 256 x 256: 35 against 24).  Fully connected layers need no walk and
+//   keep the tile kernel: 300 -> 131072 25 us against 47.
+// * 16 destinations a block while that gives every block a CU of its own
+//   (64 tiles): 784 -> 1024 5.7 us against 11, 4096 -> 4096 24 against 55,
+//   784 -> 8192 (128 tiles) 13.3 against 12.5; not for up to 64 visits,
+//   which fill an eighth of its chunk: 5 x 5 into 576 3.7 us against 6.5.
+template <int TYPE>
+static hipError_t launch_base_type(const sg_conn &c, hipStream_t st) {
+    const int tiles = (c.num_dest + 63) / 64;
+    const int count = cursor<TYPE>(c, 0).count;
+    if (TYPE != SG_FULLY_CONNECTED && tiles >= (count <= 64 ? 1024 : 2048))
+        launch_lane_type<TYPE>(c, st);
+    else if (count > 64 && tiles <= 64)
+        launch_tile_type<TYPE, 16, 16>(c, st);
+    else
+        launch_tile_type<TYPE, 64, 8>(c, st);
     return hipGetLastError();
 }
 
-// Fewer than two tiles per CU: sixteen wavefronts per tile.
 hipError_t launch_tile_base(const sg_conn &c, hipStream_t st) {
-    const int tiles = (c.num_dest + 63) / 64;
-    if (tiles < 512) return launch_tile_base_t<16, 64>(c, st);
-    return launch_tile_base_t<4, 32>(c, st);
+    switch (c.type) {
+        case SG_FULLY_CONNECTED:
+            return launch_base_type<SG_FULLY_CONNECTED>(c, st);
+        case SG_SUBSET: return launch_base_type<SG_SUBSET>(c, st);
+        case SG_CONVERGENT: return launch_base_type<SG_CONVERGENT>(c, st);
+        case SG_DIVERGENT: return launch_base_type<SG_DIVERGENT>(c, st);
+        case SG_SPARSE: return launch_base_type<SG_SPARSE>(c, st);
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_iz_tile_compact(const sg_conn &c, const sg_iz_syn &s,
