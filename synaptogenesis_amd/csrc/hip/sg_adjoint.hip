@@ -19,11 +19,10 @@
 //                          (checkpoints of at most 16 steps: both in one
 //                          launch, out_scan2_fwd, a block per batch row);
 //                          v2 of every step is kept for the backward
-//   backward  n_hid a multiple of 256 and checkpoints of at most 16
-//             steps: scan_bwd_fused, the loss gradient and all of the
-//             passes below for every block of steps in one launch (dW2
-//             summed per batch row), with pack_x as extra blocks of it;
-//             else per block, last first: layer 1's recurrence again from
+//   backward  checkpoints of at most 16 steps: scan_bwd_fused, the loss
+//             gradient and all of the passes below for every block of
+//             steps in one launch (dW2 summed per batch row), with pack_x
+//             as extra blocks of it; else per block, last first: layer 1's recurrence again from
 //             the block's checkpoint (the currents are kept), recording
 //             v1 and s1, then
 //             scan2_bwd    one thread per (b, output), steps in reverse:
@@ -92,16 +91,28 @@ __device__ __forceinline__ float act_grad_fast(float u, int mode, float slope) {
     return mode == SG_SNN_SPIKE ? g : 0.5f * slope * g;
 }
 
+// The same with one Newton step on the reciprocal (below 1 ulp again), for
+// the sizes whose passes divided exactly before they shared this scan.
+__device__ __forceinline__ float act_grad_newton(float u, int mode,
+                                                 float slope) {
+    const float d = 1.0f + slope * fabsf(u);
+    const float r0 = __builtin_amdgcn_rcpf(d);
+    const float r = fmaf(r0, fmaf(-d, r0, 1.0f), r0);
+    const float g = r * r;
+    return mode == SG_SNN_SPIKE ? g : 0.5f * slope * g;
+}
+
 // act and act_grad_fast for a mode fixed at compile time (MODE < 0: the
 // run's mode): the same operations, without the other mode's.
 template <int MODE>
 __device__ __forceinline__ float act_m(float u, int mode, float slope) {
     return act(u, MODE < 0 ? mode : MODE, slope);
 }
-template <int MODE>
+template <int MODE, bool NEWTON>
 __device__ __forceinline__ float act_grad_fast_m(float u, int mode,
                                                  float slope) {
-    return act_grad_fast(u, MODE < 0 ? mode : MODE, slope);
+    return NEWTON ? act_grad_newton(u, MODE < 0 ? mode : MODE, slope)
+                  : act_grad_fast(u, MODE < 0 ? mode : MODE, slope);
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -1235,9 +1246,9 @@ __device__ inline float loss_grad_at(const float *__restrict__ counts,
     return scale * (p - (o == labels[b] ? 1.0f : 0.0f)) / (float)B;
 }
 
-// The whole backward in one launch (n_hid a multiple of 256, checkpoints
-// of at most 16 steps): a block of 256 threads = 256 hidden units of one
-// batch row b; it walks the blocks of steps from the last, and per block
+// The whole backward in one launch (checkpoints of at most 16 steps): a
+// block of 256 threads = up to 256 hidden units of one batch row b (ANY:
+// n_hid is not a multiple of 256, so a row's last block is partly idle); it walks the blocks of steps from the last, and per block
 //  - threads o < O run layer 2's adjoint for (b, o) over the block's steps
 //    exactly as scan2_bwd does, into LDS (every block of the row computes
 //    the same values; the carry stays in a register);
@@ -1251,8 +1262,12 @@ __device__ inline float loss_grad_at(const float *__restrict__ counts,
 // fixed order).  No scan2_bwd, dw2_partial or recomputing launch.  MODE
 // (>= 0) and OUT (> 0) fix the mode and the number of outputs at compile
 // time: the per-step loops then carry no guard or select for the other
-// mode or for outputs past O.
-template <int MODE, int OUT>
+// mode or for outputs past O.  Bound by the per-step arithmetic over the a1
+// it reads and the d1 it writes: 784 -> 1024 -> 10, batch 128, 100 steps 44
+// us.  ANY against the per-block launches it replaced: a whole forward and
+// backward of 784 -> 500 -> 10, batch 50, 25 steps, 256 -> 191 us, of 333 ->
+// 777 -> 10, batch 100, 80 steps, 484 -> 262 us.
+template <int MODE, int OUT, bool ANY>
 __global__ __launch_bounds__(256) void scan_bwd_fused(
         ScanArgs a, int nblk, long slot, const uint16_t *__restrict__ w2,
         const float *__restrict__ a1, const float *__restrict__ state,
@@ -1269,11 +1284,16 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
     }
     constexpr int NO = OUT > 0 ? OUT : kMaxOut;   // output slots walked
     __shared__ float d2s[16][kMaxOut];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int H = a.H, O = OUT > 0 ? OUT : a.O;
     const long BH = (long)a.B * H, BO = (long)a.B * O;
     const long M = (long)a.steps * a.B;   // rows of a block of steps
-    const int b = i / H, u = i % H;
+    const int ub = ANY ? (H + 255) / 256 : H / 256;   // blocks of a row
+    const int b = blockIdx.x / ub;
+    const int u0 = (blockIdx.x % ub) * 256 + threadIdx.x;
+    // lanes past the row's units compute its last unit and store nothing
+    const bool live = !ANY || u0 < H;
+    const int u = ANY ? min(u0, H - 1) : u0;
+    const int i = b * H + u;
     const bool out_thread = threadIdx.x < O;
     const int i2 = b * O + (out_thread ? threadIdx.x : 0);
     const float gb = out_thread ? loss_grad_at(counts, labels, a.B, O, scale, b,
@@ -1321,7 +1341,7 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
             for (int t = 15; t >= 0; --t) {
                 if (t >= a.steps) continue;
                 const float d = (gb - a.reset_theta * dn2) *
-                                act_grad_fast_m<MODE>(v2[t] - a.theta, a.mode,
+                                act_grad_fast_m<MODE, ANY>(v2[t] - a.theta, a.mode,
                                                       a.slope) +
                                 a.beta * dn2;
                 d2s[t][threadIdx.x] = d;
@@ -1354,10 +1374,10 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
                     acc[o] = fmaf(d2s[t][o], sv, acc[o]);
                 }
             const float d = (gs - a.reset_theta * dn) *
-                            act_grad_fast_m<MODE>(vr[t] - a.theta, a.mode,
+                            act_grad_fast_m<MODE, ANY>(vr[t] - a.theta, a.mode,
                                                   a.slope) +
                             a.beta * dn;
-            lb[(long)t * BH + i] = d;
+            if (live) lb[(long)t * BH + i] = d;
             dn = d;
         }
 #pragma unroll
@@ -1367,7 +1387,7 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
     }
 #pragma unroll
     for (int o = 0; o < NO; ++o)
-        if (o < O) part2[((long)b * O + o) * H + u] = tot[o];
+        if (live && o < O) part2[((long)b * O + o) * H + u] = tot[o];
 }
 
 // Adjoint of layer 1 over one block of steps, in reverse; thread = (b, u):
@@ -1529,12 +1549,9 @@ struct Layout {
         g2, part2, part1, w2t, xp, a2all, w2f, total;
 };
 
-// The whole backward runs in one launch (scan_bwd_fused) where each
-// 256-thread block lies in one batch row and a block of steps fits its
-// LDS table of output adjoints.
-bool fused_backward(const sg_snn_cfg &c) {
-    return c.n_hid % 256 == 0 && c.checkpoint <= 16;
-}
+// The whole backward runs in one launch (scan_bwd_fused) where a block of
+// steps fits its LDS table of output adjoints.
+bool fused_backward(const sg_snn_cfg &c) { return c.checkpoint <= 16; }
 
 // dW2 partial-sum slots: one per batch row (fused backward) or per
 // kDw2Rows rows of a block of steps.
@@ -1773,11 +1790,18 @@ int sg_snn_backward(const sg_snn_cfg *cfg, const uint16_t *x,
                            float *, const uint16_t *, uint16_t *, int, int,
                            long, int);
         const bool spike = c.mode == SG_SNN_SPIKE;
-        const BK k = spike ? (O == 10 ? (BK)scan_bwd_fused<SG_SNN_SPIKE, 10>
-                                      : (BK)scan_bwd_fused<SG_SNN_SPIKE, 0>)
-                           : (O == 10 ? (BK)scan_bwd_fused<SG_SNN_RATE, 10>
-                                      : (BK)scan_bwd_fused<SG_SNN_RATE, 0>);
-        const int scan_blocks = (int)((long)B * H / 256);
+        const BK whole[2][2] = {
+            {scan_bwd_fused<SG_SNN_RATE, 0, false>,
+             scan_bwd_fused<SG_SNN_RATE, 10, false>},
+            {scan_bwd_fused<SG_SNN_SPIKE, 0, false>,
+             scan_bwd_fused<SG_SNN_SPIKE, 10, false>}};
+        const BK any[2][2] = {
+            {scan_bwd_fused<SG_SNN_RATE, 0, true>,
+             scan_bwd_fused<SG_SNN_RATE, 10, true>},
+            {scan_bwd_fused<SG_SNN_SPIKE, 0, true>,
+             scan_bwd_fused<SG_SNN_SPIKE, 10, true>}};
+        const BK k = (H % 256 == 0 ? whole : any)[spike][O == 10];
+        const int scan_blocks = B * ((H + 255) / 256);
         const long pack_blocks = blocks(gp * ((c.n_in + 7) / 8));
         hipLaunchKernelGGL(k, dim3((unsigned)(scan_blocks + pack_blocks)),
                            dim3(256), 0, s, a, nblk, slot, w2,
