@@ -311,6 +311,15 @@ int sg_hip_rate_neuron(float *input, float *output, int size, int history,
                        void *stream);
 int sg_hip_relay_neuron(float *input, float *output, int size, int history,
                         int ramp, void *stream);
+/* Rate-encoding and relay layers of a list in one launch (up to
+ * SG_MAX_FLOAT_BATCH layers per launch; longer lists are split). */
+enum { SG_RATE = 0, SG_RELAY = 1, SG_RELAY_RAMP = 2, SG_MAX_FLOAT_BATCH = 32 };
+typedef struct sg_float_layer {
+    int size, history, model;
+    const float *input;
+    float *output;                /* [history][size] */
+} sg_float_layer;
+int sg_hip_float_neurons(const sg_float_layer *layers, int n, void *stream);
 
 /* Game of life fused step for the one-connection 3x3 convolutional case:
  * activation + rule + shift in one pass over double-buffered words. */

@@ -242,26 +242,33 @@ __global__ __launch_bounds__(kNeuronBlock) void gol_neuron_kernel(
     shift_bits(output, size, nid, history, live ? 1u : 0u);
 }
 
-// re_attribute_kernel (state/impl/rate_encoding_attributes.cpp:14-23):
-// out = input > 0 ? tanh(input) : 0.  tanh is evaluated in FP64 and
-// rounded once to FP32.
-__global__ __launch_bounds__(kNeuronBlock) void rate_neuron_kernel(
-        const float *input, float *output, int size, int history) {
-    const int nid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (nid >= size) return;
-    const float in = input[nid];
-    const float v = ((double)in > 0.0) ? (float)tanh((double)in) : 0.0f;
-    shift_floats(output, size, nid, history, v);
-}
+// Up to SG_MAX_FLOAT_BATCH FLOAT layers in one grid, as IzBatch.
+struct FloatBatch {
+    int n;
+    int first[SG_MAX_FLOAT_BATCH + 1];
+    sg_float_layer l[SG_MAX_FLOAT_BATCH];
+};
 
-// relay_attribute_kernel (state/impl/relay_attributes.cpp:10-18).
-__global__ __launch_bounds__(kNeuronBlock) void relay_neuron_kernel(
-        const float *input, float *output, int size, int history, int ramp) {
-    const int nid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (nid >= size) return;
-    const float in = input[nid];
-    const float v = ramp ? (float)fmax(0.0, (double)in) : in;
-    shift_floats(output, size, nid, history, v);
+// SG_RATE: re_attribute_kernel (state/impl/rate_encoding_attributes.cpp:
+// 14-23), out = input > 0 ? tanh(input) : 0, tanh evaluated in FP64 and
+// rounded once to FP32.  SG_RELAY, SG_RELAY_RAMP: relay_attribute_kernel
+// (state/impl/relay_attributes.cpp:10-18).  A layer is a launch's worth of
+// microseconds by itself (1.3-4 us for 10 to 1024 neurons), so all of a
+// step's layers share one.
+__global__ __launch_bounds__(kNeuronBlock) void float_neuron_kernel(
+        FloatBatch f) {
+    int j = 0;
+    while (j + 1 < f.n && (int)blockIdx.x >= f.first[j + 1]) ++j;
+    const sg_float_layer &l = f.l[j];
+    const int nid = (blockIdx.x - f.first[j]) * kNeuronBlock + threadIdx.x;
+    if (nid >= l.size) return;
+    const float in = l.input[nid];
+    float v = in;
+    if (l.model == SG_RATE)
+        v = ((double)in > 0.0) ? (float)tanh((double)in) : 0.0f;
+    else if (l.model == SG_RELAY_RAMP)
+        v = (float)fmax(0.0, (double)in);
+    shift_floats(l.output, l.size, nid, l.history, v);
 }
 
 __global__ __launch_bounds__(kNeuronBlock) void set_f32_kernel(
@@ -415,22 +422,42 @@ extern "C" int sg_hip_gol_neuron(float *input, uint32_t *output, int size,
     return hipGetLastError();
 }
 
+extern "C" int sg_hip_float_neurons(const sg_float_layer *layers, int n,
+                                    void *stream) {
+    for (int s0 = 0; s0 < n; s0 += SG_MAX_FLOAT_BATCH) {
+        FloatBatch f;
+        f.n = 0;
+        int blocks = 0;
+        for (int j = s0; j < n && j < s0 + SG_MAX_FLOAT_BATCH; ++j) {
+            if (layers[j].size <= 0) continue;
+            if (layers[j].model < SG_RATE || layers[j].model > SG_RELAY_RAMP)
+                return (int)hipErrorInvalidValue;
+            f.l[f.n] = layers[j];
+            f.first[f.n] = blocks;
+            blocks += nblocks(layers[j].size);
+            ++f.n;
+        }
+        if (f.n == 0) continue;
+        f.first[f.n] = blocks;
+        hipLaunchKernelGGL(float_neuron_kernel, dim3(blocks),
+                           dim3(kNeuronBlock), 0, (hipStream_t)stream, f);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+
 extern "C" int sg_hip_rate_neuron(float *input, float *output, int size,
                                   int history, void *stream) {
-    if (size <= 0) return 0;
-    hipLaunchKernelGGL(rate_neuron_kernel, dim3(nblocks(size)),
-                       dim3(kNeuronBlock), 0, (hipStream_t)stream, input,
-                       output, size, history);
-    return hipGetLastError();
+    const sg_float_layer l = {size, history, SG_RATE, input, output};
+    return sg_hip_float_neurons(&l, 1, stream);
 }
 
 extern "C" int sg_hip_relay_neuron(float *input, float *output, int size,
                                    int history, int ramp, void *stream) {
-    if (size <= 0) return 0;
-    hipLaunchKernelGGL(relay_neuron_kernel, dim3(nblocks(size)),
-                       dim3(kNeuronBlock), 0, (hipStream_t)stream, input,
-                       output, size, history, ramp);
-    return hipGetLastError();
+    const sg_float_layer l = {size, history, ramp ? SG_RELAY_RAMP : SG_RELAY,
+                              input, output};
+    return sg_hip_float_neurons(&l, 1, stream);
 }
 
 extern "C" int sg_hip_init_random(float *p, int n, int dist, float a,

@@ -686,6 +686,7 @@ class Runner {
 
     std::map<LayerState *, InitFold> init_fold_;
     std::set<ConnState *> store_sum_;
+    std::set<LayerState *> no_clear_;   // the first activator stores
     std::map<LayerState *, std::vector<ConnState *>> tss_out_;
     std::set<ConnState *> tss_folded_;
     std::map<LayerState *, ConnState *> gol_fast_;
@@ -838,7 +839,7 @@ void Runner::setup_plans() {
     // input too, so their layers keep the separate pass.
     for (auto &lsp : st_->layers()) {
         LayerState *ls = lsp.get();
-        if (ls->model != Model::IZHIKEVICH || io_types_.count(ls) ||
+        if (ls->model != Model::IZHIKEVICH || is_input(ls) ||
             ls->layer->registers > 1)
             continue;
         InitFold f;
@@ -931,6 +932,26 @@ void Runner::setup_plans() {
         };
         dfs(ls->layer->dendrites[0].get());
         if (ls->layer->dendrites.size() > 1) any_dendrites_ = true;
+        // A layer that is only cleared before its activators: where the
+        // first to write the input covers every neuron and adds, it stores
+        // its sum instead (0 + sum has the sum's bits: a sum that starts
+        // at +0 is never -0) and the clear is not launched.
+        if (is_input(ls) || init_fold_.count(ls) || gol_fast_.count(ls) ||
+            ls->layer->registers > 1 ||
+            ls->layer->config.has_child("init config"))
+            continue;
+        ConnState *first = nullptr;
+        bool plain = true;
+        for (const Act &act : v) {
+            if (act.kind != ACT_CONN) plain = false;
+            else if (!first && is_base(*act.cs)) first = act.cs;
+        }
+        if (plain && first && first->iz_kind != SG_IZ_GAP &&
+            first->conn->opcode == SG_ADD && first->conn->type != SG_SUBSET &&
+            first->num_dest == ls->layer->size) {
+            store_sum_.insert(first);
+            no_clear_.insert(ls);
+        }
     }
 }
 
@@ -1142,7 +1163,8 @@ void Runner::activate_layer(LayerState *ls, bool split) {
 void Runner::update_neurons(const std::vector<LayerState *> &lss, int sidx,
                             const StepCtx &x) {
     std::vector<sg_iz_layer> iz_layers;
-    std::vector<Res> reads, writes;
+    std::vector<sg_float_layer> float_layers;
+    std::vector<Res> reads, writes, float_reads, float_writes;
     std::vector<ConnState *> stepped;   // time since spike stepped
     for (LayerState *ls : lss) {
         const int n = ls->layer->size;
@@ -1251,23 +1273,24 @@ void Runner::update_neurons(const std::vector<LayerState *> &lss, int sidx,
                 }
                 break;
             }
-            case Model::RATE_ENCODING: {
-                hipStream_t s = sched().begin(sidx, {rin, rout}, {rout});
-                check_hip(sg_hip_rate_neuron(ls->input.df(), ls->output.df(),
-                                             n, ls->history, s),
-                          "rate neuron");
-                sched().end();
-                break;
-            }
+            case Model::RATE_ENCODING:
             case Model::RELAY: {
-                hipStream_t s = sched().begin(sidx, {rin, rout}, {rout});
-                check_hip(sg_hip_relay_neuron(ls->input.df(), ls->output.df(),
-                                              n, ls->history, ls->ramp, s),
-                          "relay neuron");
-                sched().end();
+                const int model = ls->model == Model::RATE_ENCODING ? SG_RATE
+                                : ls->ramp ? SG_RELAY_RAMP : SG_RELAY;
+                float_layers.push_back(sg_float_layer{
+                    n, ls->history, model, ls->input.df(), ls->output.df()});
+                float_reads.insert(float_reads.end(), {rin, rout});
+                float_writes.push_back(rout);
                 break;
             }
         }
+    }
+    if (!float_layers.empty()) {
+        hipStream_t s = sched().begin(sidx, float_reads, float_writes);
+        check_hip(sg_hip_float_neurons(float_layers.data(),
+                                       (int)float_layers.size(), s),
+                  "rate and relay neurons");
+        sched().end();
     }
     if (!iz_layers.empty()) {
         hipStream_t s = sched().begin(sidx, reads, writes);
@@ -1290,7 +1313,8 @@ void Runner::pre_input(const StepCtx &x) {
         LayerState *ls = lsp.get();
         if (is_input(ls) || gol_fast_.count(ls) || in_seq_.count(ls->layer))
             continue;
-        if (!init_fold_.count(ls)) init_layer(ls, true, x);
+        if (!init_fold_.count(ls) && !no_clear_.count(ls))
+            init_layer(ls, true, x);
     }
     for (auto &lsp : layers) {
         LayerState *ls = lsp.get();
@@ -1368,7 +1392,7 @@ void Runner::post_input(const StepCtx &x) {
                 const auto ik = in_keys_.find(ls);
                 init_layer(ls, ik == in_keys_.end() ||
                                !ik->second.count("input"), x);
-            } else if (!init_fold_.count(ls)) {
+            } else if (!init_fold_.count(ls) && !no_clear_.count(ls)) {
                 init_layer(ls, true, x);
             }
             activate_layer(ls, false);

@@ -142,6 +142,7 @@ SG_STUB(sg_hip_iz_neuron, const sg_iz_layer *, void *)
 SG_STUB(sg_hip_pack_plane, const uint32_t *, int, int, uint64_t *, void *)
 SG_STUB(sg_hip_gol_neuron, float *, uint32_t *, int, int, int, int, int, int,
         void *)
+SG_STUB(sg_hip_float_neurons, const sg_float_layer *, int, void *)
 SG_STUB(sg_hip_rate_neuron, float *, float *, int, int, void *)
 SG_STUB(sg_hip_relay_neuron, float *, float *, int, int, int, void *)
 SG_STUB(sg_hip_gol_step, const uint32_t *, uint32_t *, float *, int, int, int,
