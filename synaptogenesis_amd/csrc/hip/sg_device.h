@@ -29,9 +29,22 @@ __device__ __forceinline__ void philox(uint32_t c[4], uint32_t k0,
     }
 }
 
-// ((x % n) + n) % n with C truncating %, as synapse_kernel.h:401-406.
+// ((x % n) + n) % n with C truncating %, as synapse_kernel.h:401-406; an
+// index within one layer of the edge (all but fields larger than the layer)
+// takes no division.
 __device__ __forceinline__ int wrap_index(int x, int n) {
-    return ((x % n) + n) % n;
+    const int y = x < 0 ? x + n : x >= n ? x - n : x;
+    return (unsigned)y < (unsigned)n ? y : ((x % n) + n) % n;
+}
+
+// n / d for n >= 0, d > 0 by a float quotient put right (an integer
+// division is some thirty instructions).
+__host__ __device__ __forceinline__ int quotient(int n, int d) {
+    int q = (int)((float)n * (1.0f / (float)d));
+    long r = n - (long)q * d;
+    while (r < 0) { --q; r += d; }
+    while (r >= d) { ++q; r -= d; }
+    return q;
 }
 
 // extract (engine/kernel/extractor.cpp:8-15): FLOAT reads the float,
@@ -245,7 +258,8 @@ __host__ __device__ inline SynapseCursor cursor(const sg_conn &c, int slot) {
         q.row0 = c.from_row_start; q.col0 = c.from_col_start;
         q.rstep = 1; q.cstep = 1;
     } else if (TYPE == SG_CONVERGENT) {
-        const int to_row = slot / c.to_cols, to_col = slot % c.to_cols;
+        const int to_row = quotient(slot, c.to_cols);
+        const int to_col = slot - to_row * c.to_cols;
         q.row0 = to_row * c.row_stride + c.row_spacing * c.row_offset;
         q.col0 = to_col * c.col_stride + c.col_spacing * c.col_offset;
         q.ncols = c.col_field;
@@ -256,7 +270,8 @@ __host__ __device__ inline SynapseCursor cursor(const sg_conn &c, int slot) {
         q.row0 = slot; q.col0 = 0; q.ncols = c.k_per_dest;
         q.rstep = 1; q.cstep = 1;
     } else {  // SG_DIVERGENT
-        const int to_row = slot / c.to_cols, to_col = slot % c.to_cols;
+        const int to_row = quotient(slot, c.to_cols);
+        const int to_col = slot - to_row * c.to_cols;
         q.row0 = (to_row + c.row_spacing * (-c.row_offset - c.row_field +
                                             c.row_stride)) / c.row_stride;
         q.col0 = (to_col + c.col_spacing * (-c.col_offset - c.col_field +
@@ -299,9 +314,10 @@ __device__ __forceinline__ int source_at(const sg_conn &c,
 template <int TYPE>
 struct SynapseIter {
     int k, count, kc, ncols;
-    int r, c, c0, rstep, cstep, rows, cols;
+    int r, c, r0, c0, rstep, cstep, rows, cols;
     bool wrap;
     long wi, wstep;
+    float inv;           // 1 / ncols
     const int32_t *sf;   // SG_SPARSE: the tiled source indices
 
     __device__ __forceinline__ void init(const sg_conn &cn, int slot) {
@@ -318,29 +334,39 @@ struct SynapseIter {
             // steps taken modulo the layer: one subtraction wraps a step
             rstep = wrap_index(rstep, rows); cstep = wrap_index(cstep, cols);
         }
+        r0 = r;
         c0 = c;
+        inv = 1.0f / (float)ncols;
         if (TYPE == SG_ONE_TO_ONE) { wi = slot; wstep = 0; }
         else if ((TYPE == SG_CONVERGENT || TYPE == SG_DIVERGENT) &&
                  cn.convolutional) { wi = 0; wstep = 1; }
         else { wi = tiled_index(slot, 0, cn.k_per_dest); wstep = 64; }
     }
-    // Jump to visit k (one division; then advance() walks on).
-    __device__ __forceinline__ void seek(const sg_conn &cn, int slot,
-                                         int kk) {
-        init(cn, slot);
-        if (kk <= 0 || TYPE == SG_ONE_TO_ONE) return;
-        const SynapseCursor q = cursor<TYPE>(cn, slot);
+    // From visit 0, where init() left it, to visit kk; advance() walks on.
+    // No integer division (a dozen of them cost more than eight visits'
+    // work): the row is a rounded quotient put right by one, and the wrapped
+    // steps rarely pass the layer's edge twice.
+    __device__ __forceinline__ void jump(int kk) {
         k = kk;
-        kc = kk % ncols;
-        const int kr = kk / ncols;
-        r = q.row0 + kr * q.rstep;
-        c = q.col0 + kc * q.cstep;
-        if (wrap) { r = wrap_index(r, rows); c = wrap_index(c, cols); }
         wi += (long)kk * wstep;
+        if (TYPE == SG_FULLY_CONNECTED || TYPE == SG_SPARSE ||
+            TYPE == SG_ONE_TO_ONE)
+            return;
+        int kr = (int)(((float)kk + 0.5f) * inv);
+        kc = kk - kr * ncols;
+        while (kc < 0) { --kr; kc += ncols; }
+        while (kc >= ncols) { ++kr; kc -= ncols; }
+        r = r0 + kr * rstep;
+        c = c0 + kc * cstep;
+        if (wrap) {
+            if (r >= rows) r = r < 2 * rows ? r - rows : r % rows;
+            if (c >= cols) c = c < 2 * cols ? c - cols : c % cols;
+        }
     }
     // Source index of the current visit, or -1 where the loop skips it.
     __device__ __forceinline__ int source() const {
         if (TYPE == SG_SPARSE) return sf[wi];
+        if (TYPE == SG_FULLY_CONNECTED) return k;
         if ((TYPE == SG_CONVERGENT || TYPE == SG_DIVERGENT) && !wrap &&
             (r < 0 || r >= rows || c < 0 || c >= cols))
             return -1;

@@ -11,14 +11,13 @@
 // 1. pack_plane_kernel turns the source's history words into a plane: the
 //    bit each source neuron shows this connection (word delay/32, bit
 //    31 - delay%32), 64 neurons per uint64, one wavefront ballot each.
-// 2. plane_base_kernel: a block owns a tile of 64 destinations (one lane
-//    each) and stages the plane in LDS.  Its W wavefronts split the visit
-//    list into windows of VPW * W visits: each lane tests its VPW visits'
-//    bits in LDS and issues the weight loads of the spiking ones together
-//    (coalesced across the tile), writing the weight -- or +0 for a silent
-//    or skipped visit -- to an LDS window.  After a barrier wavefront 0 adds
-//    the window in visit order.  Adding +0 leaves the sum unchanged, so the
-//    result is the reference's sum bit for bit.
+// 2. plane_base_kernel: a block stages the plane in LDS.  Its wavefronts
+//    split the visit list: each lane tests its visits' bits in LDS and
+//    issues the weight loads of the spiking ones together (coalesced across
+//    the tile), writing the weight -- or +0 for a silent or skipped visit --
+//    to an LDS chunk.  After a barrier wavefront 0 adds the chunk in visit
+//    order.  Adding +0 leaves the sum unchanged, so the result is the
+//    reference's sum bit for bit.
 //
 // Work per synapse is a bit test in LDS; weights are read only for the
 // spiking visits.  Planes larger than kPlaneMax words are read from global
@@ -30,6 +29,8 @@
 namespace sg {
 
 constexpr int kPlaneMax = 4096;     // uint64 plane words staged in LDS
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void pack_plane_kernel(
         const uint32_t *words, int n, int delay, uint64_t *plane) {
@@ -45,61 +46,107 @@ __device__ __forceinline__ int plane_visits(const sg_conn &c) {
     return cursor<TYPE>(c, 0).count;
 }
 
-template <int TYPE, int W, int VPW, int NBUF, bool STAGED>
+// D destinations a block (16 or 64, inside one tile): the chain of one
+// destination's additions bounds the launch, so it is kept off everything
+// else as in tile_base_kernel -- a chunk's weights are on their way while
+// wavefront 0 adds the chunk before, four visits to an LDS read.  Measured
+// with 5 % of the sources spiking: 15 x 15 stride 2 from 256 x 320 10.8 us
+// (13.0 before), from 32 x 40 7.1 us (9.6); 5000 -> 1000 fully connected 33
+// us (94).
+template <int TYPE, int D, int W, bool STAGED>
 __global__ __launch_bounds__(64 * W) void plane_base_kernel(
         sg_conn c, const uint64_t *plane) {
-    constexpr int WIN = VPW * W;
-    extern __shared__ uint64_t splane[];          // STAGED: the plane
-    __shared__ float vals[NBUF][WIN][64];
+    constexpr int V = 64 / D;            // visits of a wavefront load
+    constexpr int PER = 8;
+    constexpr int CHUNK = W * PER * V;
+    constexpr int AHEAD = 4;
+    static_assert(CHUNK % (4 * AHEAD) == 0, "whole reads");
+    extern __shared__ uint32_t splane[];          // STAGED: the plane
+    __shared__ f32x4 vals[2][CHUNK / 4][D];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int slot = blockIdx.x * 64 + lane;
+    const int d = lane % D, kk = lane / D;
+    const int slot = blockIdx.x * D + d;
     const bool live = slot < c.num_dest;
     const int count = plane_visits<TYPE>(c);
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(plane);
     if (STAGED) {
-        const int np = (c.from_size + 63) >> 6;
-        for (int i = threadIdx.x; i < np; i += 64 * W) splane[i] = plane[i];
+        const int np = (c.from_size + 31) >> 5;
+        for (int i = threadIdx.x; i < np; i += 64 * W) splane[i] = words[i];
+        __syncthreads();
+        words = splane;
     }
-    __syncthreads();
-    const uint64_t *pl = STAGED ? splane : plane;
     const float *wbase = c.convolutional
         ? c.weights
         : c.weights + tiled_index(live ? slot : 0, 0, c.k_per_dest);
     const long wstep = c.convolutional ? 1 : 64;
-    float sum = 0.0f;
-    for (int k0 = 0, win = 0; k0 < count; k0 += WIN, ++win) {
-        const int buf = NBUF == 2 ? (win & 1) : 0;
-        const int kw = k0 + wave * VPW;
-        if (live && kw < count) {
-            SynapseIter<TYPE> it;
-            it.seek(c, slot, kw);
-            const int n = min(VPW, count - kw);
-            float v[VPW];
+    const int first = wave * PER * V + kk;
+    SynapseIter<TYPE> start;
+    start.init(c, live ? slot : 0);
+    float v[PER];
+    auto issue = [&](int k0) {
+        SynapseIter<TYPE> it = start;
+        it.jump(k0 + first);
+        uint32_t on = 0;
 #pragma unroll
-            for (int b = 0; b < VPW; ++b) {
-                v[b] = 0.0f;
-                if (b < n) {
-                    const int from = it.source();
-                    it.advance();
-                    if (from >= 0 && ((pl[from >> 6] >> (from & 63)) & 1u))
-                        v[b] = wbase[(kw + b) * wstep];
+        for (int j = 0; j < PER; ++j) {
+            const int k = k0 + first + j * V;
+            const int from = live && k < count ? it.source() : -1;
+            if (from >= 0)
+                on |= ((words[from >> 5] >> (from & 31)) & 1u) << j;
+#pragma unroll
+            for (int b = 0; b < V; ++b) it.advance();
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            v[j] = 0.0f;
+            if ((on >> j) & 1u) v[j] = wbase[(k0 + first + j * V) * wstep];
+        }
+    };
+    auto store = [&](int buf) {
+        if (V == 1) {
+#pragma unroll
+            for (int j = 0; j < PER; j += 4) {
+                const f32x4 q = {v[j], v[j + 1], v[j + 2], v[j + 3]};
+                vals[buf][(wave * PER + j) / 4][d] = q;
+            }
+        } else {
+            float *q = reinterpret_cast<float *>(vals[buf]);
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int at = first + j * V;
+                q[((at >> 2) * D + d) * 4 + (at & 3)] = v[j];
+            }
+        }
+    };
+    float sum = 0.0f;
+    if (count > 0) {
+        issue(0);
+        store(0);
+    }
+    for (int k0 = 0, buf = 0; k0 < count; k0 += CHUNK, buf ^= 1) {
+        __syncthreads();
+        const bool more = k0 + CHUNK < count;
+        if (more) issue(k0 + CHUNK);
+        if (wave == 0) {
+            // entries past the count hold +0
+            const int groups = (min(CHUNK, count - k0) + 3) / 4;
+            for (int g = 0; g < groups; g += AHEAD) {
+                f32x4 q[AHEAD];
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) q[i] = vals[buf][g + i][d];
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) {
+                    sum += q[i][0];
+                    sum += q[i][1];
+                    sum += q[i][2];
+                    sum += q[i][3];
                 }
             }
-#pragma unroll
-            for (int b = 0; b < VPW; ++b)
-                vals[buf][wave * VPW + b][lane] = v[b];
         }
-        __syncthreads();
-        if (live && wave == 0) {
-            const int n = min(WIN, count - k0);
-            for (int j = 0; j < n; ++j) sum += vals[buf][j][lane];
-        }
-        // One buffer: the next window's writes wait for the sum.
-        if (NBUF == 1) __syncthreads();
+        if (more) store(buf ^ 1);
     }
-    if (live && wave == 0) {
-        const int to = slot_to_index(c, slot);
-        put_sum(c, to, sum);
-    }
+    if (live && wave == 0 && kk == 0)
+        put_sum(c, slot_to_index(c, slot), sum);
 }
 
 // Fully connected, at most kListMax sources: every destination visits the
@@ -148,28 +195,27 @@ __global__ __launch_bounds__(64) void fc_list_kernel(sg_conn c,
     put_sum(c, slot_to_index(c, slot), sum);
 }
 
-template <int TYPE, int W, int VPW, int NBUF>
+template <int TYPE, int D, int W>
 static hipError_t launch_plane_w(const sg_conn &c, hipStream_t st) {
-    dim3 g((c.num_dest + 63) / 64), b(64 * W);
+    dim3 g((c.num_dest + D - 1) / D), b(64 * W);
     const int np = (c.from_size + 63) / 64;
     if (np <= kPlaneMax)
-        hipLaunchKernelGGL((plane_base_kernel<TYPE, W, VPW, NBUF, true>), g,
-                           b, (size_t)np * 8, st, c, c.plane);
+        hipLaunchKernelGGL((plane_base_kernel<TYPE, D, W, true>), g, b,
+                           (size_t)np * 8, st, c, c.plane);
     else
-        hipLaunchKernelGGL((plane_base_kernel<TYPE, W, VPW, NBUF, false>), g,
-                           b, 0, st, c, c.plane);
+        hipLaunchKernelGGL((plane_base_kernel<TYPE, D, W, false>), g, b, 0,
+                           st, c, c.plane);
     return hipGetLastError();
 }
 
-// At most 16 visits per destination: one wavefront per tile, each lane
-// walks its destination's visits in order, reading the plane words through
-// the caches (no LDS staging, no barrier: a block is one short wavefront
-// that fits the single wave slot a CU has left beside a long kernel).
-// Every visit's plane word is loaded first, then the weights of the
-// spiking visits, then the sum in visit order (silent visits add +0).
+// One lane per destination: it walks its visits in order, sixteen at a
+// time, reading the plane words through the caches (no LDS staging, no
+// barrier: a block is one short wavefront).  Every visit's plane word is
+// loaded first, then the weights of the spiking visits, then the sum in
+// visit order (silent visits add +0).
 template <int TYPE>
-__global__ __launch_bounds__(64) void plane_small_kernel(sg_conn c,
-                                                         const uint64_t *plane) {
+__global__ __launch_bounds__(64) void plane_lane_kernel(sg_conn c,
+                                                        const uint64_t *plane) {
     constexpr int V = 16;
     const int slot = blockIdx.x * 64 + threadIdx.x;
     if (slot >= c.num_dest) return;
@@ -177,50 +223,59 @@ __global__ __launch_bounds__(64) void plane_small_kernel(sg_conn c,
     const float *wbase = c.convolutional
         ? c.weights : c.weights + tiled_index(slot, 0, c.k_per_dest);
     const long wstep = c.convolutional ? 1 : 64;
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(plane);
     SynapseIter<TYPE> it;
-    it.seek(c, slot, 0);
-    int from[V];
-    uint64_t word[V];
-#pragma unroll
-    for (int b = 0; b < V; ++b) {
-        from[b] = -1;
-        if (b < count) {
-            from[b] = it.source();
-            it.advance();
-        }
-        word[b] = from[b] >= 0 ? plane[from[b] >> 6] : 0ull;
-    }
-    float v[V];
-#pragma unroll
-    for (int b = 0; b < V; ++b) {
-        v[b] = 0.0f;
-        if (from[b] >= 0 && ((word[b] >> (from[b] & 63)) & 1u))
-            v[b] = wbase[b * wstep];
-    }
+    it.init(c, slot);
     float sum = 0.0f;
+    for (int k0 = 0; k0 < count; k0 += V) {
+        int from[V];
+        uint32_t word[V];
 #pragma unroll
-    for (int b = 0; b < V; ++b) sum += v[b];
+        for (int b = 0; b < V; ++b) {
+            from[b] = -1;
+            if (k0 + b < count) {
+                from[b] = it.source();
+                it.advance();
+            }
+            word[b] = from[b] >= 0 ? words[from[b] >> 5] : 0u;
+        }
+        float v[V];
+#pragma unroll
+        for (int b = 0; b < V; ++b) {
+            v[b] = 0.0f;
+            if ((word[b] >> (from[b] & 31)) & 1u)
+                v[b] = wbase[(k0 + b) * wstep];
+        }
+#pragma unroll
+        for (int b = 0; b < V; ++b) sum += v[b];
+    }
     put_sum(c, slot_to_index(c, slot), sum);
 }
 
-// A destination with at most 16 visits: plane_small_kernel.  Beside a
-// long kernel (sg_conn.beside): four wavefronts of 8 visits per tile, two
-// LDS buffers.  Otherwise sixteen wavefronts of 8 visits share a tile
-// (windows of
-// 128 visits, one LDS buffer): the most wavefronts in flight per tile,
-// which is what hides latency for the few-tile layers this path serves
-// (measured on the E/I sheet's E->I connection: 12.9 us against 19.9 us
-// with four wavefronts of 16 visits).
+// Which form (all give the same bits), by one sweep:
+// * a lane per destination for up to 16 visits, and for up to 64 once the
+//   layer's own wavefronts fill the GPU (1024 tiles): 5 x 5 on 512 x 512
+//   9.2 us against 37 with eight wavefronts a tile;
+// * 16 destinations a block while that gives every block a CU of its own
+//   (64 tiles): 15 x 15 on 64 x 64 6.9 us against 7.8;
+// * beside a long kernel on another stream (sg_conn.beside), four
+//   wavefronts a tile: they start as soon as a CU has four free wave slots;
+// * sixteen wavefronts a tile up to two tiles a CU (15 x 15 on 128 x 128
+//   7.7 us against 10 with eight), eight beyond (on 256 x 256 17.9 against
+//   19.5).
 template <int TYPE>
 static hipError_t launch_plane_t(const sg_conn &c, hipStream_t st) {
-    if (cursor<TYPE>(c, 0).count <= 16) {
-        hipLaunchKernelGGL(plane_small_kernel<TYPE>,
-                           dim3((c.num_dest + 63) / 64), dim3(64), 0, st, c,
-                           c.plane);
+    const int count = cursor<TYPE>(c, 0).count;
+    const int tiles = (c.num_dest + 63) / 64;
+    if (count <= 16 || (count <= 64 && tiles >= 1024)) {
+        hipLaunchKernelGGL(plane_lane_kernel<TYPE>, dim3(tiles), dim3(64), 0,
+                           st, c, c.plane);
         return hipGetLastError();
     }
-    if (c.beside) return launch_plane_w<TYPE, 4, 8, 2>(c, st);
-    return launch_plane_w<TYPE, 16, 8, 1>(c, st);
+    if (count > 64 && tiles <= 64) return launch_plane_w<TYPE, 16, 16>(c, st);
+    if (c.beside) return launch_plane_w<TYPE, 64, 4>(c, st);
+    if (tiles <= 512) return launch_plane_w<TYPE, 64, 16>(c, st);
+    return launch_plane_w<TYPE, 64, 8>(c, st);
 }
 
 // True when the plane path applies: a BIT source, finite weights and a

@@ -1,6 +1,5 @@
-// Tile kernels, full records: the base activator's launcher and the
-// Izhikevich passes over records with every per-synapse field; compact
-// records go to sg_tile_compact.hip.
+// Launchers of the tile kernels: the base activator, and the choice of the
+// Izhikevich passes' translation unit.
 #include "sg_tile_kernels.h"
 
 namespace sg {
@@ -77,24 +76,26 @@ hipError_t launch_tile_base(const sg_conn &c, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_iz_tile_compact(const sg_conn &c, const sg_iz_syn &s,
-                                  const sg_iz_dest &d, int kind, int sub,
-                                  int upd, int act, const float *st_,
+// launch_iz_tile_<compact record><sixteen wavefronts a tile> (sg_tile_iz.h)
+#define SG_DECLARE(N)                                                        \
+    hipError_t launch_iz_tile_##N(const sg_conn &c, const sg_iz_syn &s,      \
+                                  const sg_iz_dest &d, int kind, int sub,    \
+                                  int upd, int act, const float *st_,        \
                                   const float *dt_, hipStream_t st);
+SG_DECLARE(00)
+SG_DECLARE(01)
+SG_DECLARE(10)
+SG_DECLARE(11)
+#undef SG_DECLARE
 
 hipError_t launch_iz_tile(const sg_conn &c, const sg_iz_syn &s,
                           const sg_iz_dest &d, int kind, int sub, int upd,
                           int act, const float *st_, const float *dt_,
                           hipStream_t st) {
-    if (s.src_stp)
-        return launch_iz_tile_compact(c, s, d, kind, sub, upd, act, st_, dt_,
-                                      st);
-    if (upd && act)
-        return launch_iz_tile_t<1, 1, 0>(c, s, d, kind, sub, st_, dt_, st);
-    if (upd)
-        return launch_iz_tile_t<1, 0, 0>(c, s, d, sub ? SG_IZ_SUB : SG_IZ_ADD,
-                                         sub, st_, dt_, st);
-    return launch_iz_tile_t<0, 1, 0>(c, s, d, kind, 0, st_, dt_, st);
+    const bool wide = wide_tiles((c.num_dest + 63) / 64);
+    auto *launch = s.src_stp ? (wide ? launch_iz_tile_11 : launch_iz_tile_10)
+                             : (wide ? launch_iz_tile_01 : launch_iz_tile_00);
+    return launch(c, s, d, kind, sub, upd, act, st_, dt_, st);
 }
 
 }  // namespace sg

@@ -8,9 +8,8 @@
 // SUBSET, CONVERGENT, DIVERGENT): the base activator and the three
 // Izhikevich synapse passes (update, activate, fused update+activate).
 //
-// A block owns a tile of 64 destinations.  Its W wavefronts (W = 3 or 4
-// for the Izhikevich passes, chosen per launch so that the whole grid is
-// resident at once where possible) split the tile's synapse list k-wise in
+// A block owns a tile of 64 destinations.  Its W wavefronts (W = 3, 4 or 16
+// for the Izhikevich passes, chosen per launch) split the tile's synapse list k-wise in
 // chunks of 8 * W (8 visits per wavefront per chunk): every synapse's
 // independent work -- loads, STDP / short-term plasticity, trace decay,
 // stores -- runs with W wavefronts in flight per tile instead of one.  The
@@ -48,26 +47,25 @@ __device__ __forceinline__ int visit_count(const sg_conn &c) {
 // ---------------------------------------------------------------------------
 // Base activator (synapse_kernel.h:887-912) of sources that are not spike
 // planes.
-template <int TYPE>
-__device__ __forceinline__ void ordered_sum_n(const float (*vals)[64],
-                                              SynapseIter<TYPE> &walk, int n,
-                                              int lane, float &sum) {
-    for (int j = 0; j < n; ++j) {
-        const bool valid = walk.source() >= 0;
-        walk.advance();
-        if (valid) sum += vals[j][lane];
-    }
-}
-
-// The same sum where every skipped visit wrote +0.0f (SPARSE: a slot's
-// visits past its own nonzero count).  Adding +0.0f leaves every value but
-// -0.0f unchanged (quiet NaNs keep their payload), and a sum that starts at
-// +0.0f is never -0.0f (x + y rounds to -0.0f only when both are -0.0f), so
-// the result is bit for bit the sum over the valid visits alone -- without
-// reading each visit's source index again.
+// The sum of a chunk's n visits in visit order, where every skipped visit
+// (outside a layer that does not wrap, past a SPARSE slot's own nonzero
+// count) wrote +0.0f.  Adding +0.0f leaves every value but -0.0f unchanged
+// (quiet NaNs keep their payload), and a sum that starts at +0.0f is never
+// -0.0f (x + y rounds to -0.0f only when both are -0.0f), so the result is
+// bit for bit the sum over the valid visits alone -- without walking the
+// visits again.
 __device__ __forceinline__ void dense_sum_n(const float (*vals)[64], int n,
                                             int lane, float &sum) {
-    for (int j = 0; j < n; ++j) sum += vals[j][lane];
+    int j = 0;
+    // sixteen reads on their way before the additions wait for the first
+    for (; j + 16 <= n; j += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = vals[j + i][lane];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum += v[i];
+    }
+    for (; j < n; ++j) sum += vals[j][lane];
 }
 
 // A block owns D destinations (16 or 64, inside one tile); a wavefront load
@@ -106,20 +104,18 @@ __global__ __launch_bounds__(64 * WAVES) void tile_base_kernel(sg_conn c) {
     bool on[PER];
     // Starts the loads of the chunk at k0; a visit without a source reads
     // visit 0 of source 0 and is dropped when it is stored.
+    SynapseIter<TYPE> start;
+    start.init(c, live ? slot : 0);
     auto issue = [&](int k0) {
-        SynapseIter<TYPE> it;
-        if (TYPE != SG_FULLY_CONNECTED) it.seek(c, live ? slot : 0, k0 + first);
+        SynapseIter<TYPE> it = start;
+        it.jump(k0 + first);
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int k = k0 + first + j * V;
             int from = -1;
-            if (TYPE == SG_FULLY_CONNECTED) {
-                from = k < count ? k : -1;
-            } else {
-                if (k < count) from = it.source();
+            if (k < count) from = it.source();
 #pragma unroll
-                for (int b = 0; b < V; ++b) it.advance();
-            }
+            for (int b = 0; b < V; ++b) it.advance();
             on[j] = live && from >= 0;
             x[j] = c.src[on[j] ? from : 0];
             if (!skip) w[j] = wbase[on[j] ? k * wstep : 0];
@@ -335,15 +331,15 @@ __global__ __launch_bounds__(64 * WAVES) void iz_tile_kernel(
         sure = c.tile_counts[2 * blockIdx.x];
         count = c.tile_counts[2 * blockIdx.x + 1];
     }
-    SynapseIter<TYPE> walk;
-    walk.init(c, live ? slot : 0);
+    SynapseIter<TYPE> start;
+    start.init(c, live ? slot : 0);
     float sum = 0.0f;
     for (int k0 = 0, chunk = 0; k0 < count; k0 += CHUNK, ++chunk) {
         const int buf = chunk & 1;
         const int kw = k0 + wave * kPerWave;
         if (live && kw < count) {
-            SynapseIter<TYPE> it;
-            it.seek(c, slot, kw);
+            SynapseIter<TYPE> it = start;
+            it.jump(kw);
             // Record of visit kw (a multiple of 8) of this lane's
             // destination: group kw / 8 of tile blockIdx.x; visit kw + b is
             // b * F * 64 further, its delay byte b * 64 further.
@@ -401,8 +397,8 @@ __global__ __launch_bounds__(64 * WAVES) void iz_tile_kernel(
 #pragma unroll
             for (int b = 0; b < kSub; ++b) {
                 if (CHECK && from[b] < 0) {
-                    // SPARSE: the ordered sum adds every visit of the chunk
-                    if (TYPE == SG_SPARSE && ACT) {
+                    // the ordered sum adds every visit of the chunk
+                    if (ACT) {
                         vals[buf][0][wave * kPerWave + h + b][lane] = 0.0f;
                         if (kLong)
                             vals[buf][1][wave * kPerWave + h + b][lane] = 0.0f;
@@ -465,12 +461,8 @@ __global__ __launch_bounds__(64 * WAVES) void iz_tile_kernel(
         if (ACT) {
             __syncthreads();
             if (live && (wave == 0 || (kLong && wave == 1))) {
-                const int n = min(CHUNK, count - k0);
-                // SPARSE: skipped visits wrote +0.0f (see dense_sum_n)
-                if (k0 + n <= sure || TYPE == SG_SPARSE)
-                    dense_sum_n(vals[buf][wave], n, lane, sum);
-                else
-                    ordered_sum_n(vals[buf][wave], walk, n, lane, sum);
+                dense_sum_n(vals[buf][wave], min(CHUNK, count - k0), lane,
+                            sum);
             }
         }
     }
@@ -500,10 +492,15 @@ static inline int cu_count() {
     return cached[dev];
 }
 
-// Wavefronts per tile for a fused Izhikevich launch: the count that lets
-// the whole grid be resident in the fewest rounds of blocks (a grid that
-// overflows the GPU by a fraction runs its last round mostly idle), ties
-// going to more wavefronts per tile.
+// Wavefronts per tile for an Izhikevich launch over `tiles` tiles.  Up to a
+// tile per CU: sixteen (the WIDE instantiations), two chunks for a 15 x 15
+// arbor instead of eight and as many memory latencies less: 20 tiles 12 us
+// against 20 with four (260 tiles with sixteen would run a second round:
+// 130 x 128 56 us a step, 128 x 128 45).  Beyond that three or four, whichever lets the whole grid be resident in the fewest rounds of
+// blocks (a grid that overflows the GPU by a fraction runs its last round
+// mostly idle), ties going to four.
+static inline bool wide_tiles(int tiles) { return tiles <= cu_count(); }
+
 template <class KA, class KB>
 static inline int pick_waves(KA *four, KB *three, int tiles) {
     int nb4 = 0, nb3 = 0;
@@ -519,7 +516,7 @@ static inline int pick_waves(KA *four, KB *three, int tiles) {
     return r3 < r4 ? 3 : 4;
 }
 
-template <int UPD, int ACT, int COMPACT>
+template <int UPD, int ACT, int COMPACT, bool WIDE>
 hipError_t launch_iz_tile_t(const sg_conn &c, const sg_iz_syn &s,
                                    const sg_iz_dest &d, int kind, int sub,
                                    const float *st_, const float *dt_,
@@ -528,12 +525,20 @@ hipError_t launch_iz_tile_t(const sg_conn &c, const sg_iz_syn &s,
     dim3 g(tiles);
 #define SG_IZ(T, K, S)                                                       \
     do {                                                                     \
-        auto *k4 = iz_tile_kernel<T, K, S, UPD, ACT, 4, COMPACT>;            \
-        auto *k3 = iz_tile_kernel<T, K, S, UPD, ACT, 3, COMPACT>;            \
-        if (pick_waves(k4, k3, tiles) == 3)                                  \
-            hipLaunchKernelGGL(k3, g, dim3(192), 0, st, c, s, d, st_, dt_);  \
-        else                                                                 \
-            hipLaunchKernelGGL(k4, g, dim3(256), 0, st, c, s, d, st_, dt_);  \
+        if constexpr (WIDE) {                                                \
+            hipLaunchKernelGGL((iz_tile_kernel<T, K, S, UPD, ACT, 16,        \
+                                COMPACT>), g, dim3(1024), 0, st, c, s, d,    \
+                               st_, dt_);                                    \
+        } else {                                                             \
+            auto *k4 = iz_tile_kernel<T, K, S, UPD, ACT, 4, COMPACT>;        \
+            auto *k3 = iz_tile_kernel<T, K, S, UPD, ACT, 3, COMPACT>;        \
+            if (pick_waves(k4, k3, tiles) == 3)                              \
+                hipLaunchKernelGGL(k3, g, dim3(192), 0, st, c, s, d, st_,    \
+                                   dt_);                                     \
+            else                                                             \
+                hipLaunchKernelGGL(k4, g, dim3(256), 0, st, c, s, d, st_,    \
+                                   dt_);                                     \
+        }                                                                    \
     } while (0)
 #define SG_IZK(T, S)                                                         \
     switch (kind) {                                                          \
