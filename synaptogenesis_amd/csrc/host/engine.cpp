@@ -958,18 +958,24 @@ void Runner::setup_plans() {
 // ---- streams ----------------------------------------------------------------
 // One stream per structure (engine/cluster/cluster.cpp:9-16,
 // parallel_cluster.cpp:27-40 give each layer of a cluster a compute stream
-// and the cluster an IO stream; here a structure is the unit); in a
-// parallel structure whose layers have both kinds of activators, the ones
-// that write a layer's input (base activators, gap junctions) on a second
-// stream of their own, beside the conductance passes (which write
-// conductances and synapse records).  The environment's copies run on
-// the stream of their layer.  Kernel timing keeps everything on stream 0.
+// and the cluster an IO stream; here a structure is the unit).  The
+// environment's copies run on the stream of their layer.  With "concurrent
+// activators": "true", in a parallel structure whose layers have both kinds
+// of activators the ones that write a layer's input (base activators, gap
+// junctions) run on a second stream, beside the conductance passes (which
+// write conductances and synapse records).  Not by default: the events
+// between the streams cost more than the overlap saves on all but the
+// largest networks, and where several states' streams share the hardware
+// queues also there.  E/I sheets, us a step with one stream and with two:
+// 32x40 33 / 50, 128x128 45 / 56, 256x320 137 / 134 alone and 147 / 152
+// with three states in turn (sparse: 128 / 155).  Kernel timing keeps
+// everything on stream 0.
 void Runner::setup_streams() {
     const bool one = kt_.on;
     const bool per_structure = !one &&
                                args_.get_bool("structure streams", true);
     const bool concurrent = !one &&
-                            args_.get_bool("concurrent activators", true);
+                            args_.get_bool("concurrent activators", false);
     int next = 0;
     const auto &structs = net_->structures();
     for (size_t si = 0; si < structs.size(); ++si)
