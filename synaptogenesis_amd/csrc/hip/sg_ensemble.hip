@@ -590,6 +590,37 @@ int layer_tiles(int precision, int R) {
                                     : (R + kTileRows - 1) / kTileRows;
 }
 
+// The launch shape of an ensemble that is not given one (sg_ens_set_tile,
+// sg_ens_autotune), from a sweep of every shape, us a step:
+//   8 instances of 128..512 (358 row tiles)    1x8 4.0  2x4 4.0  4x1 5.1
+//   1 of 2048 (256)                            1x8 6.2  2x4 7.3  4x1 13.1
+//   64 of 128..1024 (4863)                     2x2 17.4 2x4 18.0 4x1 17.7
+//   64 of 64..256 (1375)                       2x2 4.2  2x4 4.1  4x1 5.4
+//   16 of 1024..2048 (3179)                    2x4 28.7 2x2 30.0 4x1 30.8
+//   256 of 128..4096 (69920)                   2x4 701  2x2 706  4x1 705
+// Up to two row tiles a CU a step is one wavefront's walk of the fan-in, so
+// eight share it; beyond that blocks of two row tiles start and end more
+// evenly than blocks of four, and long rows are split over four wavefronts.
+// FP32: eight row groups a block (8 instances 4.65 us against 4.80 with
+// four, 1 of 2048 9.0 against 10.9).
+void default_shape(sg_ens *e) {
+    long tiles = 0, k = 0;
+    for (const Layer &l : e->layers) {
+        tiles += l.tiles;
+        k += (long)l.tiles * l.Kp;
+    }
+    if (e->precision == SG_ENS_FP32) {
+        e->rt = 8;
+        e->ks = 1;
+    } else if (tiles <= 512) {
+        e->rt = 1;
+        e->ks = 8;
+    } else {
+        e->rt = 2;
+        e->ks = k >= 1024 * tiles ? 4 : 2;
+    }
+}
+
 size_t layer_weight_bytes(int precision, int R, int Kp) {
     if (precision == SG_ENS_FP32)
         return (size_t)ceil_to(R, kGroupRows) * Kp * 4;
@@ -629,8 +660,6 @@ sg_ens *sg_ens_create(int n, const int *widths, int precision, float leak,
     e->seed = seed;
     e->workload = workload;
     e->widths.assign(widths, widths + 3 * n);
-    e->rt = precision == SG_ENS_FP32 ? 4 : 4;
-    e->ks = 1;
     auto bail = [&](int) { sg_ens_destroy(e); return (sg_ens *)nullptr; };
     // state: x0, h1[2], h2[2] per instance, each padded to 32 floats
     long off = 0;
@@ -710,6 +739,7 @@ sg_ens *sg_ens_create(int n, const int *widths, int precision, float leak,
         fail("ensemble initialisation failed");
         return bail(0);
     }
+    default_shape(e);
     if (build_items(e)) return bail(0);
     return e;
 }
