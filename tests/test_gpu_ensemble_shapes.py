@@ -36,3 +36,40 @@ def test_default_shape(widths, precision, shape):
         e.close()
     for a, b in zip(*states):
         assert np.abs(a - b).max() <= 1e-5 * max(1e-3, np.abs(b).max())
+
+
+@pytest.mark.gpu
+def test_reads_follow_every_change():
+    """Enough reads bring the whole state over at once; runs, writes, timing
+    and tuning in between must show, whichever way a read is served."""
+    widths = [[40, 70, 33], [5, 64, 100], [17, 3, 9]]
+    e = RateEnsemble(widths, "bf16", leak=0.5)
+    f = RateEnsemble(widths, "bf16", leak=0.5)
+
+    def every(a):
+        return [a.state(i, k) for i in range(3) for k in range(3)]
+
+    def alone():
+        # a single read a run: never from the mirror
+        out = []
+        for i in range(3):
+            for k in range(3):
+                f.set_state(0, 0, f.state(0, 0))
+                out.append(f.state(i, k))
+        return out
+
+    for step in range(4):
+        for a in (e, f):
+            a.run(1 + step, graph=step % 2 == 0)
+        for _ in range(3):
+            for x, y in zip(every(e), alone()):
+                assert np.array_equal(x, y)
+        new = np.linspace(0, 1, 70, dtype=np.float32) * step
+        for a in (e, f):
+            a.set_state(0, 1, new)
+        assert np.array_equal(every(e)[1], new)
+        e.autotune(1)
+        f.set_tile(*e.tile)
+        assert np.array_equal(every(e)[1], new)
+    e.close()
+    f.close()
