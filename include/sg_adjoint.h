@@ -82,6 +82,22 @@ int sg_snn_backward(const sg_snn_cfg *cfg, const uint16_t *x,
                     const int32_t *labels, void *workspace, float grad_scale,
                     float *dw1, float *dw2, void *stream);
 
+/* The same with FP32 weights, rounded to BF16 (nearest even) into w1b
+ * [n_hid][n_in] and w2b [n_out][n_hid], which the backward takes. */
+int sg_snn_forward_fp32(const sg_snn_cfg *cfg, const uint16_t *x,
+                        const float *w1, const float *w2, uint16_t *w1b,
+                        uint16_t *w2b, const int32_t *labels, void *workspace,
+                        float *loss, float *counts, void *stream);
+
+/* sg_snn_backward with grad_scale 1 whose gradients are multiplied by *grad,
+ * a float on the device (the incoming gradient of the loss), as they are
+ * written. */
+int sg_snn_backward_times(const sg_snn_cfg *cfg, const uint16_t *x,
+                          const uint16_t *w1, const uint16_t *w2,
+                          const int32_t *labels, void *workspace,
+                          const float *grad, float *dw1, float *dw2,
+                          void *stream);
+
 const char *sg_snn_error(void);
 
 #ifdef __cplusplus

@@ -88,6 +88,10 @@ def library():
     L.sg_snn_forward.restype = ctypes.c_int
     L.sg_snn_backward.argtypes = [cp, P, P, P, P, P, ctypes.c_float, P, P, P]
     L.sg_snn_backward.restype = ctypes.c_int
+    L.sg_snn_forward_fp32.argtypes = [cp, P, P, P, P, P, P, P, P, P, P]
+    L.sg_snn_forward_fp32.restype = ctypes.c_int
+    L.sg_snn_backward_times.argtypes = [cp, P, P, P, P, P, P, P, P, P]
+    L.sg_snn_backward_times.restype = ctypes.c_int
     L.sg_snn_error.restype = ctypes.c_char_p
     _lib = L
     return L
@@ -166,6 +170,20 @@ def validate(x, w1, w2, labels, cfg):
         _checked_labels[key] = version
 
 
+def _plain_pointer(grad, device):
+    """The address of the loss's incoming gradient where the library can
+    multiply by it: one float on `device`, and no product that autograd has
+    to record (create_graph) or to batch (a tensor without storage)."""
+    import torch
+    if (torch.is_grad_enabled() or grad.dtype != torch.float32 or
+            grad.device != device or grad.numel() != 1):
+        return None
+    try:
+        return ctypes.c_void_p(grad.data_ptr())
+    except RuntimeError:
+        return None
+
+
 def _function():
     import torch
 
@@ -175,8 +193,15 @@ def _function():
         @staticmethod
         def forward(ctx, x, w1, w2, labels, cfg):
             validate(x, w1, w2, labels, cfg)
-            w1b = w1.detach().to(torch.bfloat16).contiguous()
-            w2b = w2.detach().to(torch.bfloat16).contiguous()
+            # FP32 weights are rounded by one launch of the library
+            fp32 = w1.dtype == w2.dtype == torch.float32
+            if fp32:
+                w1, w2 = w1.contiguous(), w2.contiguous()
+                w1b = torch.empty_like(w1, dtype=torch.bfloat16)
+                w2b = torch.empty_like(w2, dtype=torch.bfloat16)
+            else:
+                w1b = w1.detach().to(torch.bfloat16).contiguous()
+                w2b = w2.detach().to(torch.bfloat16).contiguous()
             x = x.contiguous()
             labels = labels.contiguous()
             ws = torch.empty(workspace_bytes(cfg), dtype=torch.uint8,
@@ -184,9 +209,16 @@ def _function():
             loss = torch.empty((), dtype=torch.float32, device=x.device)
             counts = torch.empty(cfg.batch, cfg.n_out, dtype=torch.float32,
                                  device=x.device)
-            _check(library().sg_snn_forward(
-                ctypes.byref(cfg), _ptr(x), _ptr(w1b), _ptr(w2b),
-                _ptr(labels), _ptr(ws), _ptr(loss), _ptr(counts), _stream()))
+            if fp32:
+                _check(library().sg_snn_forward_fp32(
+                    ctypes.byref(cfg), _ptr(x), _ptr(w1), _ptr(w2),
+                    _ptr(w1b), _ptr(w2b), _ptr(labels), _ptr(ws),
+                    _ptr(loss), _ptr(counts), _stream()))
+            else:
+                _check(library().sg_snn_forward(
+                    ctypes.byref(cfg), _ptr(x), _ptr(w1b), _ptr(w2b),
+                    _ptr(labels), _ptr(ws), _ptr(loss), _ptr(counts),
+                    _stream()))
             ctx.save_for_backward(x, w1b, w2b, labels, ws)
             ctx.cfg = cfg
             ctx.mark_non_differentiable(counts)
@@ -200,6 +232,13 @@ def _function():
                               device=x.device)
             dw2 = torch.empty(cfg.n_out, cfg.n_hid, dtype=torch.float32,
                               device=x.device)
+            grad = _plain_pointer(grad_loss, x.device)
+            if grad is not None:
+                _check(library().sg_snn_backward_times(
+                    ctypes.byref(cfg), _ptr(x), _ptr(w1b), _ptr(w2b),
+                    _ptr(labels), _ptr(ws), grad, _ptr(dw1), _ptr(dw2),
+                    _stream()))
+                return None, dw1, dw2, None, None
             _check(library().sg_snn_backward(
                 ctypes.byref(cfg), _ptr(x), _ptr(w1b), _ptr(w2b),
                 _ptr(labels), _ptr(ws), ctypes.c_float(1.0), _ptr(dw1),

@@ -613,7 +613,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_fwd_dma(
 // extra blocks of the dW1 product's launch).
 __device__ __forceinline__ void dw2_reduce_block(
         const float *__restrict__ part, float *__restrict__ dw2, int chunks,
-        int H, int O, int blk) {
+        int H, int O, const float *__restrict__ scale, int blk) {
     __shared__ float q[4][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = blk * 64 + lane;
@@ -638,7 +638,8 @@ __device__ __forceinline__ void dw2_reduce_block(
     q[w][lane] = acc;
     __syncthreads();
     if (w == 0 && i < O * H)
-        dw2[i] = ((q[0][lane] + q[1][lane]) + q[2][lane]) + q[3][lane];
+        dw2[i] = (((q[0][lane] + q[1][lane]) + q[2][lane]) + q[3][lane]) *
+                 (scale ? *scale : 1.0f);
     __syncthreads();   // q is reused by the block's next output group
 }
 
@@ -657,7 +658,7 @@ __global__ __launch_bounds__(256) void gemm_dw1_dma(
         const float *__restrict__ L, const uint16_t *__restrict__ xp,
         float *__restrict__ part, int M, int H, int K, int per, long gp,
         const float *__restrict__ part2, float *__restrict__ dw2, int chunks2,
-        int O) {
+        int O, const float *__restrict__ scale) {
     __shared__ __align__(16) float L0[kDr * kDh], L1[kDr * kDh],
         L2[kDr * kDh];
     __shared__ __align__(16) uint16_t X0[8 * 512], X1[8 * 512], X2[8 * 512];
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(256) void gemm_dw1_dma(
         // the last z slice sums dW2 (dw2_reduce's work) beside the product
         const int ng = (O * H + 63) / 64;
         for (int g = bx + nx * by; g < ng; g += nx * ny)
-            dw2_reduce_block(part2, dw2, chunks2, H, O, g);
+            dw2_reduce_block(part2, dw2, chunks2, H, O, scale, g);
         return;
     }
     const int h0 = by * kDh, kb = bx * kDk;
@@ -774,10 +775,11 @@ __global__ __launch_bounds__(256) void gemm_dw1_dma(
         }
 }
 
-// D[i] = part[0][i] + part[1][i] + ... in range order, four at a time
-// where n and D allow it.
+// D[i] = part[0][i] + part[1][i] + ... in range order, times *scale (or 1),
+// four at a time where n and D allow it.
 __global__ void add_parts(const float *__restrict__ part, float *__restrict__ D,
-                          long n, int parts) {
+                          long n, int parts, const float *__restrict__ scale) {
+    const float g = scale ? *scale : 1.0f;
     const long n4 = (n % 4 == 0 && ((uintptr_t)D & 15) == 0) ? n / 4 : 0;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n4;
          i += (long)gridDim.x * blockDim.x) {
@@ -789,13 +791,17 @@ __global__ void add_parts(const float *__restrict__ part, float *__restrict__ D,
             acc.z += v.z;
             acc.w += v.w;
         }
+        acc.x *= g;
+        acc.y *= g;
+        acc.z *= g;
+        acc.w *= g;
         ((float4 *)D)[i] = acc;
     }
     for (long i = 4 * n4 + blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
          i += (long)gridDim.x * blockDim.x) {
         float acc = part[i];
         for (int z = 1; z < parts; ++z) acc += part[(long)z * n + i];
-        D[i] = acc;
+        D[i] = acc * g;
     }
 }
 
@@ -1471,8 +1477,8 @@ __global__ void dw2_partial(const float *__restrict__ g2,
 
 __global__ __launch_bounds__(256) void dw2_reduce(
         const float *__restrict__ part, float *__restrict__ dw2, int chunks,
-        int H, int O) {
-    dw2_reduce_block(part, dw2, chunks, H, O, blockIdx.x);
+        int H, int O, const float *__restrict__ scale) {
+    dw2_reduce_block(part, dw2, chunks, H, O, scale, blockIdx.x);
 }
 
 // Mean softmax cross-entropy over the batch (one block; sums in batch
@@ -1519,6 +1525,22 @@ __global__ void loss_grad_kernel(const float *__restrict__ counts,
     if (b >= B) return;
     for (int o = 0; o < O; ++o)
         g[b * O + o] = loss_grad_at(counts, labels, B, O, scale, b, o);
+}
+
+// FP32 weights to BF16, nearest even (a NaN stays one): both layers' in one
+// launch, the second after the first.
+__global__ void round_weights(const float *__restrict__ w1,
+                              const float *__restrict__ w2,
+                              uint16_t *__restrict__ w1b,
+                              uint16_t *__restrict__ w2b, long n1, long n2) {
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n1 + n2;
+         i += (long)gridDim.x * blockDim.x) {
+        const float v = i < n1 ? w1[i] : w2[i - n1];
+        const uint16_t b =
+            v != v ? (uint16_t)0x7FC0u : (uint16_t)bf16_rne(v);
+        if (i < n1) w1b[i] = b;
+        else w2b[i - n1] = b;
+    }
 }
 
 __global__ void fill_kernel(float *p, long n, float v) {
@@ -1754,10 +1776,11 @@ int sg_snn_forward(const sg_snn_cfg *cfg, const uint16_t *x,
     return 0;
 }
 
-int sg_snn_backward(const sg_snn_cfg *cfg, const uint16_t *x,
+static int backward(const sg_snn_cfg *cfg, const uint16_t *x,
                     const uint16_t *w1, const uint16_t *w2,
                     const int32_t *labels, void *workspace, float grad_scale,
-                    float *dw1, float *dw2, void *stream) {
+                    const float *grad, float *dw1, float *dw2,
+                    void *stream) {
     if (check(cfg)) return 1;
     if (!x || !w1 || !w2 || !labels || !workspace || !dw1 || !dw2)
         return fail("null pointer");
@@ -1839,18 +1862,52 @@ int sg_snn_backward(const sg_snn_cfg *cfg, const uint16_t *x,
         // one more z slice of blocks sums dW2
         const dim3 g2(dgrid.x, dgrid.y, kTnSplit + 1);
         hipLaunchKernelGGL(gemm_dw1_dma, g2, dim3(256), 0, s, lam, xp, part1,
-                           MT, H, c.n_in, per, gp, part2, dw2, chunks, O);
+                           MT, H, c.n_in, per, gp, part2, dw2, chunks, O, grad);
     } else {
         hipLaunchKernelGGL(gemm_dw1, dgrid, dim3(256), 0, s, lam, xp, part1,
                            MT, H, c.n_in, per);
         hipLaunchKernelGGL(dw2_reduce, dim3((O * H + 63) / 64), dim3(256), 0,
-                           s, part2, dw2, chunks, H, O);
+                           s, part2, dw2, chunks, H, O, grad);
     }
     hipLaunchKernelGGL(add_parts, dim3(1024), dim3(256), 0, s, part1, dw1,
-                       (long)H * c.n_in, kTnSplit);
+                       (long)H * c.n_in, kTnSplit, grad);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(std::string("launch: ") + hipGetErrorString(e));
     return 0;
+}
+
+int sg_snn_backward(const sg_snn_cfg *cfg, const uint16_t *x,
+                    const uint16_t *w1, const uint16_t *w2,
+                    const int32_t *labels, void *workspace, float grad_scale,
+                    float *dw1, float *dw2, void *stream) {
+    return backward(cfg, x, w1, w2, labels, workspace, grad_scale, nullptr,
+                    dw1, dw2, stream);
+}
+
+int sg_snn_backward_times(const sg_snn_cfg *cfg, const uint16_t *x,
+                          const uint16_t *w1, const uint16_t *w2,
+                          const int32_t *labels, void *workspace,
+                          const float *grad, float *dw1, float *dw2,
+                          void *stream) {
+    if (!grad) return fail("null pointer");
+    return backward(cfg, x, w1, w2, labels, workspace, 1.0f, grad, dw1, dw2,
+                    stream);
+}
+
+int sg_snn_forward_fp32(const sg_snn_cfg *cfg, const uint16_t *x,
+                        const float *w1, const float *w2, uint16_t *w1b,
+                        uint16_t *w2b, const int32_t *labels, void *workspace,
+                        float *loss, float *counts, void *stream) {
+    if (check(cfg)) return 1;
+    if (!x || !w1 || !w2 || !w1b || !w2b || !labels || !workspace || !loss)
+        return fail("null pointer");
+    const long n1 = (long)cfg->n_hid * cfg->n_in;
+    const long n2 = (long)cfg->n_out * cfg->n_hid;
+    const unsigned g = blocks(n1 + n2);
+    hipLaunchKernelGGL(round_weights, dim3(g < 4096 ? g : 4096), dim3(256), 0,
+                       (hipStream_t)stream, w1, w2, w1b, w2b, n1, n2);
+    return sg_snn_forward(cfg, x, w1b, w2b, labels, workspace, loss, counts,
+                          stream);
 }
 
 }  // extern "C"
