@@ -325,6 +325,100 @@ __device__ __forceinline__ uint64_t gol_from_next_lane(uint64_t v) {
     return (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
 }
 
+// Any function of three bit masks by its truth table (the table's bit for
+// inputs x, y, z is bit 4x + 2y + z).
+template <uint32_t TABLE>
+__device__ __forceinline__ uint64_t gol_bits3(uint64_t x, uint64_t y,
+                                              uint64_t z) {
+    const uint32_t lo = __builtin_amdgcn_bitop3_b32(
+        (uint32_t)x, (uint32_t)y, (uint32_t)z, TABLE);
+    const uint32_t hi = __builtin_amdgcn_bitop3_b32(
+        (uint32_t)(x >> 32), (uint32_t)(y >> 32), (uint32_t)(z >> 32), TABLE);
+    return (uint64_t)hi << 32 | lo;
+}
+constexpr uint32_t kXor3 = 0x96, kMajority = 0xE8, kOneOf3 = 0x16,
+                   kNoneOf3 = 0x01, kChoose = 0xCA, kAndOr = 0xE0;
+
+// One step of the game of life's own rule (eight neighbours, survival on
+// 2-3, birth on 3) for a line of 64 cells per lane, b its newest bits and p
+// its survival bits (alive 32 steps back): the sums of three along the line
+// by a full adder, the neighbour lines' from the neighbour lanes, their
+// total as a ones mask and four twos masks (cnt).  The count is 2 or 3 where
+// exactly one twos mask is set, and the cell lives there if the ones mask or
+// its survival bit is set.  Three-input bit operations and 32-bit funnel
+// shifts: 40 instructions where the two-input form, which summed all three
+// lines in every lane with 64-bit shifts, took 90 (1024 x 1024, 8 steps a
+// launch on words: 8.4 -> 7.6 us).
+__device__ __forceinline__ uint64_t gol_life(uint64_t b, uint64_t p,
+                                             uint64_t (&cnt)[5]) {
+    const uint32_t lo = (uint32_t)b, hi = (uint32_t)(b >> 32);
+    const uint64_t up =
+        (uint64_t)__builtin_amdgcn_alignbit(hi, lo, 31) << 32 | lo << 1;
+    const uint64_t dn =
+        (uint64_t)(hi >> 1) << 32 | __builtin_amdgcn_alignbit(hi, lo, 1);
+    const uint64_t s3 = gol_bits3<kXor3>(up, b, dn);
+    const uint64_t c3 = gol_bits3<kMajority>(up, b, dn);
+    const uint64_t sa = gol_from_prev_lane(s3), ca = gol_from_prev_lane(c3);
+    const uint64_t sd = gol_from_next_lane(s3), cd = gol_from_next_lane(c3);
+    const uint64_t sb = up ^ dn, cb = up & dn;
+    const uint64_t one = gol_bits3<kXor3>(sa, sb, sd);
+    const uint64_t c1 = gol_bits3<kMajority>(sa, sb, sd);
+    const uint64_t t1 = gol_bits3<kChoose>(c1, gol_bits3<kNoneOf3>(ca, cb, cd),
+                                           gol_bits3<kOneOf3>(ca, cb, cd));
+    cnt[0] = one;
+    cnt[1] = ca;
+    cnt[2] = cb;
+    cnt[3] = cd;
+    cnt[4] = c1;
+    return gol_bits3<kAndOr>(t1, one, p);
+}
+
+// The newest bits of a row of 64 cells after one step, lane = row: gol_life,
+// or for other 0/1 kernels and rules the count of 64 cells at once as four
+// bit planes in cnt (a ripple add of each weighted neighbour mask) and the
+// rule as the union of the count's equality masks for the values the
+// survival and birth ranges admit.
+template <bool LIFE, int NP>
+__device__ __forceinline__ uint64_t gol_rule(uint64_t b, uint64_t p,
+                                             uint32_t wmask, uint32_t surv,
+                                             uint32_t birth,
+                                             uint64_t (&cnt)[NP]) {
+    if constexpr (LIFE) return gol_life(b, p, cnt);
+    // rows above and below by whole-wavefront DPP shifts (every lane
+    // active); the edge rows get 0, which only touches the rows no output
+    // depends on
+    const uint64_t a = gol_from_prev_lane(b), d = gol_from_next_lane(b);
+    const uint64_t nbr[9] = {a << 1, a, a >> 1, b << 1, b,
+                             b >> 1, d << 1, d, d >> 1};
+    uint64_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        if (!((wmask >> q) & 1u)) continue;
+        const uint64_t x = nbr[q];
+        const uint64_t k0 = c0 & x;
+        c0 ^= x;
+        const uint64_t k1 = c1 & k0;
+        c1 ^= k0;
+        const uint64_t k2 = c2 & k1;
+        c2 ^= k1;
+        c3 |= k2;
+    }
+    uint64_t sv = 0, bv = 0;
+#pragma unroll
+    for (int v = 0; v <= 9; ++v) {
+        if (!(((surv | birth) >> v) & 1u)) continue;
+        const uint64_t eq = ((v & 1) ? c0 : ~c0) & ((v & 2) ? c1 : ~c1) &
+                            ((v & 4) ? c2 : ~c2) & ((v & 8) ? c3 : ~c3);
+        if ((surv >> v) & 1u) sv |= eq;
+        if ((birth >> v) & 1u) bv |= eq;
+    }
+    cnt[0] = c0;
+    cnt[1] = c1;
+    cnt[2] = c2;
+    cnt[3] = c3;
+    return (p & sv) | (~p & bv);
+}
+
 // Kernels whose nine weights are each 0 or 1 (the game of life's own:
 // ones around a cleared centre): K steps (1 <= K <= 8) on rows of 64 cells
 // packed into 64-bit masks.  A block owns a 64 x 64 region of cells (rows
@@ -337,14 +431,7 @@ __device__ __forceinline__ uint64_t gol_from_next_lane(uint64_t v) {
 // for step s) and, on a bounded board, the cells inside it, by ballot; lane
 // j of the wavefront collects row j's masks.  One wavefront then takes all
 // K steps, lane i = region row i, with the rows above and below from its
-// neighbour lanes.  LIFE (neighbours = the eight around the cell, survival
-// on 2-3, birth on 3): each row's horizontal sums by full adders, their sum
-// as a ones mask and four twos masks; the count is 2 or 3 where exactly one
-// twos mask is set, and the cell lives there if the ones mask or its
-// survival bit is set.  Otherwise the count of 64 cells at once as four bit
-// planes (a ripple add of each weighted neighbour mask) and the rule as the
-// union of the count's equality masks for the values the survival and
-// birth ranges admit.  The count equals the integer sum of the one-weighted
+// neighbour lanes (gol_rule).  The count equals the integer sum of the one-weighted
 // bits, which is the float sum of the one-step kernel exactly; cells
 // outside a bounded board hold 0 at every step.  Finally each wavefront
 // writes its rows' inner words: the staged word shifted by K with the K new
@@ -425,69 +512,12 @@ __global__ __launch_bounds__(64 * W) void gol_packed_kernel(
         const uint64_t ib = staged[1][lane];
 #pragma unroll
         for (int s = 0; s < K; ++s) {
-            // rows above and below by whole-wavefront DPP shifts (every
-            // lane active); the edge rows get 0, which only touches the
-            // rows no output depends on
-            const uint64_t a = gol_from_prev_lane(b);
-            const uint64_t d = gol_from_next_lane(b);
             const uint64_t p = staged[2 + s][lane];
-            if (LIFE) {
-                const uint64_t al = a << 1, ar = a >> 1, bl = b << 1,
-                               br = b >> 1, dl = d << 1, dr = d >> 1;
-                uint64_t t = al ^ a;
-                const uint64_t sa = t ^ ar, ca = (al & a) | (ar & t);
-                const uint64_t sb = bl ^ br, cb = bl & br;
-                t = dl ^ d;
-                const uint64_t sd = t ^ dr, cd = (dl & d) | (dr & t);
-                t = sa ^ sb;
-                const uint64_t one = t ^ sd, c1 = (sa & sb) | (sd & t);
-                // count = one + 2 (ca + cb + cd + c1): 2 or 3 where exactly
-                // one of the four twos masks is set
-                const uint64_t p1 = ca ^ cb, q1 = cd ^ c1;
-                const uint64_t t1 =
-                    (p1 ^ q1) & ~((ca & cb) | (cd & c1) | (p1 & q1));
-                b = t1 & (one | p) & ib;
-                if (s == K - 1 && input) {
-                    planes[0][lane] = one;
-                    planes[1][lane] = ca;
-                    planes[2][lane] = cb;
-                    planes[3][lane] = cd;
-                    planes[NP - 1][lane] = c1;
-                }
-            } else {
-                const uint64_t nbr[9] = {a << 1, a, a >> 1, b << 1, b,
-                                         b >> 1, d << 1, d, d >> 1};
-                uint64_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+            uint64_t cnt[NP];
+            b = gol_rule<LIFE>(b, p, wmask, surv, birth, cnt) & ib;
+            if (s == K - 1 && input) {
 #pragma unroll
-                for (int q = 0; q < 9; ++q) {
-                    if (!((wmask >> q) & 1u)) continue;
-                    const uint64_t x = nbr[q];
-                    const uint64_t k0 = c0 & x;
-                    c0 ^= x;
-                    const uint64_t k1 = c1 & k0;
-                    c1 ^= k0;
-                    const uint64_t k2 = c2 & k1;
-                    c2 ^= k1;
-                    c3 |= k2;
-                }
-                uint64_t sv = 0, bv = 0;
-#pragma unroll
-                for (int v = 0; v <= 9; ++v) {
-                    if (!(((surv | birth) >> v) & 1u)) continue;
-                    const uint64_t eq = ((v & 1) ? c0 : ~c0) &
-                                        ((v & 2) ? c1 : ~c1) &
-                                        ((v & 4) ? c2 : ~c2) &
-                                        ((v & 8) ? c3 : ~c3);
-                    if ((surv >> v) & 1u) sv |= eq;
-                    if ((birth >> v) & 1u) bv |= eq;
-                }
-                b = ((p & sv) | (~p & bv)) & ib;
-                if (s == K - 1 && input) {
-                    planes[0][lane] = c0;
-                    planes[1][lane] = c1;
-                    planes[2][lane] = c2;
-                    planes[3][lane] = c3;
-                }
+                for (int q = 0; q < NP; ++q) planes[q][lane] = cnt[q];
             }
             halves[lane][0][s] = (uint32_t)b;
             halves[lane][1][s] = (uint32_t)(b >> 32);
@@ -607,28 +637,11 @@ __global__ __launch_bounds__(64) void gol_column_kernel(
     }
     uint64_t b = (uint64_t)nhi << 32 | nlo;
     uint64_t step[K];
-    uint64_t one = 0, ca = 0, cb = 0, cd = 0, c1 = 0;
+    uint64_t cnt[5] = {0, 0, 0, 0, 0};
 #pragma unroll
     for (int s = 0; s < K; ++s) {
-        const uint64_t L = gol_from_prev_lane(b);   // the column left
-        const uint64_t R = gol_from_next_lane(b);   // the column right
-        const uint64_t p = (uint64_t)khi[s] << 32 | klo[s];
-        const uint64_t lu = L << 1, ld = L >> 1, bu = b << 1, bd = b >> 1,
-                       ru = R << 1, rd = R >> 1;
-        uint64_t t = lu ^ L;
-        const uint64_t sa = t ^ ld;
-        ca = (lu & L) | (ld & t);
-        const uint64_t sb = bu ^ bd;
-        cb = bu & bd;
-        t = ru ^ R;
-        const uint64_t sd = t ^ rd;
-        cd = (ru & R) | (rd & t);
-        t = sa ^ sb;
-        one = t ^ sd;
-        c1 = (sa & sb) | (sd & t);
-        const uint64_t p1 = ca ^ cb, q1 = cd ^ c1;
-        const uint64_t t1 = (p1 ^ q1) & ~((ca & cb) | (cd & c1) | (p1 & q1));
-        b = t1 & (one | p) & ib;
+        // the columns left and right from the neighbour lanes
+        b = gol_life(b, (uint64_t)khi[s] << 32 | klo[s], cnt) & ib;
         step[s] = b;
     }
     if (lane < K || lane >= 64 - K || c >= cols) return;
@@ -653,15 +666,212 @@ __global__ __launch_bounds__(64) void gol_column_kernel(
         const long idx = (long)(row0 + r) * cols + c;
         __builtin_nontemporal_store(word, &out[idx]);
         if (input)
-            input[idx] = (float)((int)((one >> r) & 1ull) +
-                                 2 * ((int)((ca >> r) & 1ull) +
-                                      (int)((cb >> r) & 1ull) +
-                                      (int)((cd >> r) & 1ull) +
-                                      (int)((c1 >> r) & 1ull)));
+            input[idx] = (float)((int)((cnt[0] >> r) & 1ull) +
+                                 2 * ((int)((cnt[1] >> r) & 1ull) +
+                                      (int)((cnt[2] >> r) & 1ull) +
+                                      (int)((cnt[3] >> r) & 1ull) +
+                                      (int)((cnt[4] >> r) & 1ull)));
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Long runs of kernels of 0s and 1s: the board as bit planes.
+//
+// A word's 32 bits are the cell's last 32 states, so a step that works on
+// words moves all of them to add one.  Here each time step is a plane of its
+// own, a bit per cell, in a ring of kGolRing slots: a step reads the newest
+// plane and the one from 32 steps back and writes one, 3/8 B a cell instead
+// of 8, and nothing is shifted, packed or unpacked between launches.  The
+// words are turned into planes before a run's steps and back after them.
+//
+// Plane layout: 32-column words, word column outermost, [ceil(cols / 32)]
+// [row], so that the 64 lanes of a wavefront (one row each) read 256
+// consecutive bytes; rows padded to a multiple of four (gol_pitch); bits past
+// the last column are 0.
+constexpr int kGolRing = 48;    // 32 states and the 16 a launch writes
+
+__host__ __device__ __forceinline__ int gol_pitch(int rows) {
+    return (rows + 3) / 4 * 4;
+}
+
+// 32 x 32 bits across the lanes of each half wavefront (lane i = row i, bit
+// k = column k) transposed in five exchanges.
+__device__ __forceinline__ uint32_t gol_transpose32(uint32_t x, int lane) {
+#pragma unroll
+    for (int j = 16; j > 0; j >>= 1) {
+        // the bits whose index has no j: 0x0000ffff, 0x00ff00ff, ...
+        const uint32_t m = 0xffffffffu / ((1u << j) + 1u);
+        const uint32_t t = (uint32_t)__shfl_xor((int)x, j);
+        x = (lane & j) ? (x & ~m) | ((t & ~m) >> j)
+                       : (x & m) | ((t & m) << j);
+    }
+    return x;
+}
+
+// words -> planes in slots 0 .. 31 (oldest first; bit 0 of a word is its
+// oldest state), and back from the 32 slots that end at `newest`.  A
+// wavefront takes 64 columns of four rows.
+__global__ __launch_bounds__(64) void gol_to_planes(
+        const uint32_t *__restrict__ words, uint32_t *__restrict__ ring,
+        int rows, int cols) {
+    const int lane = threadIdx.x, half = lane >> 5, b = lane & 31;
+    const int c = blockIdx.x * 64 + lane, r0 = blockIdx.y * 4;
+    const int W = (cols + 31) / 32, pitch = gol_pitch(rows);
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        v[j] = c < cols && r0 + j < rows ? words[(long)(r0 + j) * cols + c]
+                                         : 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = gol_transpose32(v[j], lane);
+    const int wc = blockIdx.x * 2 + half;
+    if (wc < W)
+        *reinterpret_cast<uint4 *>(
+            &ring[((long)b * W + wc) * pitch + r0]) =
+            make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+__global__ __launch_bounds__(64) void gol_from_planes(
+        const uint32_t *__restrict__ ring, uint32_t *__restrict__ words,
+        int rows, int cols, int newest) {
+    const int lane = threadIdx.x, half = lane >> 5, b = lane & 31;
+    const int c = blockIdx.x * 64 + lane, r0 = blockIdx.y * 4;
+    const int W = (cols + 31) / 32, pitch = gol_pitch(rows);
+    const int slot = (newest + kGolRing - 31 + b) % kGolRing;
+    const int wc = blockIdx.x * 2 + half;
+    uint4 q = make_uint4(0u, 0u, 0u, 0u);
+    if (wc < W)
+        q = *reinterpret_cast<const uint4 *>(
+            &ring[((long)slot * W + wc) * pitch + r0]);
+    uint32_t v[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = gol_transpose32(v[j], lane);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (c < cols && r0 + j < rows)
+            __builtin_nontemporal_store(v[j],
+                                        &words[(long)(r0 + j) * cols + c]);
+}
+
+// K steps (at most 16) from the plane in slot `newest`.  A wavefront owns 32
+// columns of 64 - 2K rows: lane = row, each row's 64 cells around those
+// columns as one mask, K rows and 16 columns of halo; every step's new bits
+// are exact one cell further in.  All of the planes' words are on their way
+// before the first is used: read one window after another they were two
+// thirds of a launch (1024 x 1024, 16 steps: 13.1 -> 5.6 us).  Bound by the
+// steps' instruction chain on small boards and by their issue on large ones:
+// 1024 x 1024 0.35 us a step (0.95 on words), 4096 x 4096 1.6 us (5.3),
+// 16384 x 16384 29 us (64).
+template <int K, bool LIFE>
+__global__ __launch_bounds__(64) void gol_plane_kernel(
+        uint32_t *ring, int rows, int cols, int wrap, int newest,
+        uint32_t wmask, uint32_t surv, uint32_t birth) {
+    static_assert(K <= 16, "the halo of a word column");
+    const int lane = threadIdx.x;
+    const int W = (cols + 31) / 32, pitch = gol_pitch(rows);
+    const long plane = (long)W * pitch;
+    const int wc = blockIdx.x, x0 = wc * 32;
+    const int r = blockIdx.y * (64 - 2 * K) - K + lane;
+    const int rr = wrap ? gol_wrap_k(r, rows) : min(max(r, 0), rows - 1);
+    const bool row_in = wrap || (r >= 0 && r < rows);
+    // the words left and right of the column's; a wrapping board whose last
+    // word is partly filled is put together at its edges bit by bit
+    const bool ragged = wrap && cols % 32 != 0 &&
+                        (wc == 0 || x0 + 48 > cols);
+    const int lw = wc > 0 ? wc - 1 : W - 1, rw = wc + 1 < W ? wc + 1 : 0;
+    const bool lin = wrap || wc > 0, rin = wrap || wc + 1 < W;
+    // slots of the planes read: the survival planes, then the newest
+    auto read_slot = [&](int i) {
+        const int n = i == K ? newest : newest + 17 + i;
+        return n < kGolRing ? n : n - kGolRing;
+    };
+    uint64_t read[K + 1];
+    if (!ragged) {
+        // every word on its way before the first is used
+        uint32_t l[K + 1], m[K + 1], h[K + 1];
+#pragma unroll
+        for (int i = 0; i <= K; ++i) {
+            const uint32_t *p = ring + read_slot(i) * plane + rr;
+            l[i] = p[(long)lw * pitch];
+            m[i] = p[(long)wc * pitch];
+            h[i] = p[(long)rw * pitch];
+        }
+#pragma unroll
+        for (int i = 0; i <= K; ++i)
+            read[i] = (uint64_t)(lin ? l[i] >> 16 : 0u) |
+                      (uint64_t)m[i] << 16 |
+                      (uint64_t)(rin ? h[i] : 0u) << 48;
+    } else {
+#pragma unroll
+        for (int i = 0; i <= K; ++i) read[i] = 0;
+        int col = ((x0 - 16) % cols + cols) % cols;
+        for (int at = 0; at < 64;) {
+            const int n = min(min(64 - at, cols - col), 32 - (col & 31));
+            const uint64_t keep = ((uint64_t)1 << n) - 1;
+            const uint32_t *p = ring + rr + (long)(col >> 5) * pitch;
+            uint32_t w[K + 1];
+#pragma unroll
+            for (int i = 0; i <= K; ++i) w[i] = p[read_slot(i) * plane];
+#pragma unroll
+            for (int i = 0; i <= K; ++i)
+                read[i] |= ((uint64_t)(w[i] >> (col & 31)) & keep) << at;
+            at += n;
+            col += n;
+            if (col >= cols) col = 0;
+        }
+    }
+    uint64_t b = read[K];
+    // cells outside a bounded board hold 0 at every step
+    uint64_t inside = ~(uint64_t)0;
+    if (!wrap) {
+        if (x0 < 16) inside &= ~(uint64_t)0 << (16 - x0);
+        if (x0 + 48 > cols) inside &= ~(uint64_t)0 >> (x0 + 48 - cols);
+        if (!row_in) inside = 0;
+        b &= inside;
+    }
+    const uint32_t kept = x0 + 32 <= cols
+        ? 0xffffffffu : (1u << (cols - x0)) - 1u;
+    uint32_t made[K];
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+        uint64_t cnt[LIFE ? 5 : 4];
+        b = gol_rule<LIFE>(b, read[s], wmask, surv, birth, cnt) & inside;
+        made[s] = (uint32_t)(b >> 16);
+    }
+    if (lane < K || lane >= 64 - K || r >= rows) return;
+    int slot = newest;
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+        if (++slot == kGolRing) slot = 0;
+        ring[slot * plane + (long)wc * pitch + r] = made[s] & kept;
     }
 }
 
 }  // namespace sg
+
+namespace {
+
+// Weights of 0 and 1 as flags (bit q = weight q); false for any other.
+bool bit_weights(const float *k, uint32_t &mask) {
+    mask = 0;
+    for (int q = 0; q < 9; ++q) {
+        if (k[q] == 1.0f) mask |= 1u << q;
+        else if (k[q] != 0.0f) return false;   // -0.0f counts as 0
+    }
+    return true;
+}
+
+// Rule ranges as flags over the counts 0 .. 9.
+void rule_flags(int smin, int smax, int bmin, int bmax, uint32_t &surv,
+                uint32_t &birth) {
+    surv = birth = 0;
+    for (int v = 0; v <= 9; ++v) {
+        if (v >= smin && v <= smax) surv |= 1u << v;
+        if (v >= bmin && v <= bmax) birth |= 1u << v;
+    }
+}
+
+}  // namespace
 
 extern "C" int sg_hip_gol_step(const uint32_t *words_in, uint32_t *words_out,
                                float *input, int rows, int cols, int wrap,
@@ -711,18 +921,9 @@ extern "C" int sg_hip_gol_steps(const uint32_t *words_in, uint32_t *words_out,
     if (rows <= 0 || cols <= 0) return 0;
     // weights of 0 and 1 only: the packed form
     uint32_t wmask = 0;
-    bool bitw = true;
-    for (int q = 0; q < 9; ++q) {
-        if (k[q] == 1.0f) wmask |= 1u << q;
-        else if (k[q] != 0.0f) bitw = false;   // -0.0f counts as 0
-    }
-    if (bitw) {
-        // rule ranges as flags over the counts 0 .. 9
+    if (bit_weights(k, wmask)) {
         uint32_t surv = 0, birth = 0;
-        for (int v = 0; v <= 9; ++v) {
-            if (v >= smin && v <= smax) surv |= 1u << v;
-            if (v >= bmin && v <= bmax) birth |= 1u << v;
-        }
+        rule_flags(smin, smax, bmin, bmax, surv, birth);
         const int ti = 64 - 2 * steps;
         const dim3 g((cols + ti - 1) / ti, (rows + ti - 1) / ti);
         typedef void (*PK)(const uint32_t *, uint32_t *, float *, int, int,
@@ -795,5 +996,52 @@ extern "C" int sg_hip_gol_steps(const uint32_t *words_in, uint32_t *words_out,
                        words_in, words_out, input, rows, cols, wrap, k[0],
                        k[1], k[2], k[3], k[4], k[5], k[6], k[7], k[8], smin,
                        smax, bmin, bmax);
+    return hipGetLastError();
+}
+
+// Steps of a plane launch: sixteen up to four wavefronts a SIMD, where a
+// launch costs its chain rather than its halo (a cell computed four times),
+// eight beyond (2.7 times).
+static int plane_steps(int rows, int cols) {
+    const long waves16 = (long)((cols + 31) / 32) * ((rows + 31) / 32);
+    return waves16 <= 4096 ? 16 : 8;
+}
+
+extern "C" long sg_hip_gol_planes_bytes(const float *k, int rows, int cols) {
+    uint32_t wmask;
+    if (rows <= 0 || cols <= 0 || !bit_weights(k, wmask)) return 0;
+    return (long)sg::kGolRing * ((cols + 31) / 32) * sg::gol_pitch(rows) * 4;
+}
+
+extern "C" int sg_hip_gol_planes(const uint32_t *words_in,
+                                 uint32_t *words_out, uint32_t *planes,
+                                 int rows, int cols, int wrap, const float *k,
+                                 int smin, int smax, int bmin, int bmax,
+                                 int steps, int *launches, void *stream) {
+    using namespace sg;
+    uint32_t wmask, surv, birth;
+    if (steps < 1 || steps % 16 != 0 || !bit_weights(k, wmask))
+        return (int)hipErrorInvalidValue;
+    if (rows <= 0 || cols <= 0) return 0;
+    rule_flags(smin, smax, bmin, bmax, surv, birth);
+    const bool life = wmask == 0x1efu && surv == 0xcu && birth == 0x8u;
+    hipStream_t st = (hipStream_t)stream;
+    const dim3 turn((cols + 63) / 64, (rows + 3) / 4);
+    hipLaunchKernelGGL(gol_to_planes, turn, dim3(64), 0, st, words_in, planes,
+                       rows, cols);
+    const int K = plane_steps(rows, cols), ti = 64 - 2 * K;
+    const dim3 g((cols + 31) / 32, (rows + ti - 1) / ti);
+    auto *kern = K == 16
+        ? (life ? gol_plane_kernel<16, true> : gol_plane_kernel<16, false>)
+        : (life ? gol_plane_kernel<8, true> : gol_plane_kernel<8, false>);
+    int newest = 31;
+    for (int t = 0; t < steps; t += K) {
+        hipLaunchKernelGGL(kern, g, dim3(64), 0, st, planes, rows, cols, wrap,
+                           newest, wmask, surv, birth);
+        newest = (newest + K) % kGolRing;
+    }
+    hipLaunchKernelGGL(gol_from_planes, turn, dim3(64), 0, st, planes,
+                       words_out, rows, cols, newest);
+    if (launches) *launches = steps / K + 2;
     return hipGetLastError();
 }

@@ -227,6 +227,8 @@ struct Cache : EngineCache {
     Sched sched;
     // second word buffer of each game-of-life layer on the fused step
     std::map<LayerState *, uint32_t *> gol_spare;
+    // bit planes of a game-of-life layer's long runs (null: no memory)
+    std::map<LayerState *, uint32_t *> gol_planes;
     // step counter that captured steps read their random draws' step from
     uint64_t *d_step = nullptr;
     uint64_t *h_step = nullptr;     // pinned staging for it
@@ -234,6 +236,7 @@ struct Cache : EngineCache {
     ~Cache() override {
         graphs.clear();
         for (auto &kv : gol_spare) (void)hipFree(kv.second);
+        for (auto &kv : gol_planes) (void)hipFree(kv.second);
         if (d_step) (void)hipFree(d_step);
         if (h_step) (void)hipHostFree(h_step);
     }
@@ -700,6 +703,12 @@ class Runner {
     std::map<LayerState *, int> gol_ahead_;
     long gol_rem_ = 1;
     long gol_launches_ = 0;
+    // With more than this many steps left a layer of a 0/1 kernel takes them
+    // as bit planes, at most so many at once (an interrupt waits for them):
+    // turning a 1024 x 1024 board into planes and back costs about what 16
+    // steps on words do, and the planes halve the rest.
+    static constexpr long kGolPlanesFrom = 128, kGolPlanesMost = 4096;
+    uint32_t *gol_planes_of(LayerState *ls, const float *k9);
     bool gol_pending() const {
         for (const auto &kv : gol_ahead_)
             if (kv.second > 0) return true;
@@ -1166,6 +1175,22 @@ void Runner::activate_layer(LayerState *ls, bool split) {
     }
 }
 
+// The layer's bit planes, kept with the state; null where its kernel does
+// not have them or the device has no room.
+uint32_t *Runner::gol_planes_of(LayerState *ls, const float *k9) {
+    const long bytes = sg_hip_gol_planes_bytes(k9, ls->layer->rows,
+                                               ls->layer->cols);
+    if (bytes <= 0) return nullptr;
+    auto it = C_->gol_planes.find(ls);
+    if (it != C_->gol_planes.end()) return it->second;
+    uint32_t *p = nullptr;
+    if (hipMalloc((void **)&p, (size_t)bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    return C_->gol_planes[ls] = p;
+}
+
 void Runner::update_neurons(const std::vector<LayerState *> &lss, int sidx,
                             const StepCtx &x) {
     std::vector<sg_iz_layer> iz_layers;
@@ -1249,6 +1274,32 @@ void Runner::update_neurons(const std::vector<LayerState *> &lss, int sidx,
                     const bool last = k == 1 ? x.last
                                              : iterations_ != 0 && k == gol_rem_;
                     uint32_t *spare = C_->gol_spare.at(ls);
+                    uint32_t *planes = nullptr;
+                    if (gol_multi_.count(ls) && gol_rem_ > kGolPlanesFrom)
+                        planes = gol_planes_of(ls, k9);
+                    if (planes) {
+                        // all but the last steps, which write the input
+                        const int n = (int)std::min<long>(
+                            gol_rem_ - 1, kGolPlanesMost) / 16 * 16;
+                        int launches = 0;
+                        hipStream_t s = sched().begin(
+                            sidx, {rout, res(RES_SYN, gf->second)}, {rout});
+                        kt_.time("gol_planes", [&] {
+                            check_hip(sg_hip_gol_planes(
+                                          ls->output.du(), ls->output.du(),
+                                          planes, ls->layer->rows,
+                                          ls->layer->cols,
+                                          gf->second->conn->arbor.wrap, k9,
+                                          ls->survival_min, ls->survival_max,
+                                          ls->birth_min, ls->birth_max, n,
+                                          &launches, s),
+                                      "gol planes");
+                        });
+                        sched().end();
+                        ahead = n - 1;
+                        gol_launches_ += launches;
+                        break;
+                    }
                     hipStream_t s = sched().begin(
                         sidx, {rout, rin, res(RES_SYN, gf->second)},
                         {rout, rin});

@@ -149,6 +149,11 @@ SG_STUB(sg_hip_gol_step, const uint32_t *, uint32_t *, float *, int, int, int,
         const float *, int, int, int, int, void *)
 SG_STUB(sg_hip_gol_steps, const uint32_t *, uint32_t *, float *, int, int,
         int, const float *, int, int, int, int, int, void *)
+SG_STUB(sg_hip_gol_planes, const uint32_t *, uint32_t *, uint32_t *, int, int,
+        int, const float *, int, int, int, int, int, int *, void *)
+long sg_hip_gol_planes_bytes(const float *, int rows, int cols) {
+    return 6L * rows * cols + 64;
+}
 int sg_hip_gol_max_steps(const float *k, int rows, int cols) {
     for (int q = 0; q < 9; ++q)
         if (k[q] != 0.0f && k[q] != 1.0f) return 4;
