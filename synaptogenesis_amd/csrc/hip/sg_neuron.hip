@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "sg_device.h"
 #include "sg_hip.h"
@@ -145,12 +146,20 @@ __device__ __forceinline__ void iz_step(const sg_iz_layer &l, int nid) {
             t_rev[t][6] = r1.z; t_rev[t][7] = r1.w;
         }
 
-        for (int i = 0; i < 10 && (double)voltage < 30.0; ++i) {
+        // One of up to ten Euler steps.  PLAIN: no conductances, see below.
+        const double divisor = 1.0 + 0.1 * (double)(ampa + nmda + gabaa +
+                                                    gabab);
+        auto euler = [&](auto plain) {
+            constexpr bool PLAIN = decltype(plain)::value;
             float current = -ampa * voltage;
-            // powf(x, 2) is folded to x * x by the reference's compiler.
-            const float x = (voltage + 80.0f) / 60.0f;
-            const float temp = x * x;
-            current = current - nmda * (temp / (1.0f + temp)) * voltage;
+            float factor = 0.0f;
+            if (!PLAIN) {
+                // powf(x, 2) is folded to x * x by the reference's compiler.
+                const float x = (voltage + 80.0f) / 60.0f;
+                const float temp = x * x;
+                factor = temp / (1.0f + temp);
+            }
+            current = current - nmda * factor * voltage;
             current = current - gabaa * (voltage + 70.0f);
             current = current - gabab * (voltage + 90.0f);
             current = current * (1.0f + mult);
@@ -161,10 +170,9 @@ __device__ __forceinline__ void iz_step(const sg_iz_layer &l, int nid) {
                               (double)recovery + (double)current;
             const float delta_v = (float)dv;
 
-            const float sum_g = ampa + nmda + gabaa + gabab;
             const float drive = delta_v + (gabaa * -70.0f) + (gabab * -90.0f);
-            voltage = (float)(((double)voltage + 0.1 * (double)drive) /
-                              (1.0 + 0.1 * (double)sum_g));
+            const double moved = (double)voltage + 0.1 * (double)drive;
+            voltage = (float)(PLAIN ? moved : moved / divisor);
             voltage = (voltage != voltage) ? 30.0f : voltage;
 
             const float adjusted_tau = ((double)voltage > 30.0)
@@ -172,7 +180,22 @@ __device__ __forceinline__ void iz_step(const sg_iz_layer &l, int nid) {
                           (30.0 - (double)voltage + (double)delta_v) * 0.1)
                 : (float)0.1;
             recovery = recovery + a * adjusted_tau * ((b * voltage) - recovery);
-        }
+        };
+        // The loop is one dependent chain of about a hundred instructions,
+        // and with a wavefront a SIMD the launch is that chain.  Where no
+        // neuron of the wavefront has conductances its three divisions, a
+        // third of it and the slowest, have known results: +0 times the
+        // NMDA factor is +0 (the factor is in [0, 1] while the voltage's
+        // square does not overflow), and x / 1.0 is x.  Two layers of 1000
+        // without conductances: 9.45 -> 8.92 us a step.
+        int i = 0;
+        if (__all(__float_as_uint(nmda) == 0u && divisor == 1.0))
+            for (; i < 10 && (double)voltage < 30.0; ++i) {
+                if (!__all(fabsf(voltage) < 1e18f)) break;
+                euler(std::true_type{});
+            }
+        for (; i < 10 && (double)voltage < 30.0; ++i)
+            euler(std::false_type{});
 
         l.ampa[nid] = 0.0f;
         l.nmda[nid] = 0.0f;
