@@ -399,6 +399,15 @@ int sg_hip_copy32(const void *src, void *dst, long n, void *stream);
  * environment I/O: a kernel in the consuming stream's order instead of a
  * DMA copy on a stream of its own and the events between them. */
 int sg_hip_copy_u32(const void *src, void *dst, long n, void *stream);
+/* Several such copies in one launch (up to SG_MAX_COPY_BATCH per launch;
+ * longer lists are split). */
+enum { SG_MAX_COPY_BATCH = 32 };
+typedef struct sg_copy {
+    const void *src;
+    void *dst;
+    long n;
+} sg_copy;
+int sg_hip_copies_u32(const sg_copy *copies, int n, void *stream);
 
 /* Device properties: number of visible devices, -1 on error. */
 int sg_hip_device_count(void);

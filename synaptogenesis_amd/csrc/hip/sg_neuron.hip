@@ -387,13 +387,25 @@ __global__ __launch_bounds__(kNeuronBlock) void copy32_kernel(
         dst[i] = src[i];
 }
 
-// Any n: 16-byte words where both sides allow it, then the tail.
-__global__ __launch_bounds__(kNeuronBlock) void copy_u32_kernel(
-        const uint32_t *src, uint32_t *dst, long n, int vec) {
-    const long stride = (long)gridDim.x * blockDim.x;
-    const long i0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// Any n: 16-byte words where both sides allow it, then the tail.  Copy j of
+// the batch has blocks first[j] .. first[j + 1] - 1.
+struct CopyBatch {
+    int n;
+    int first[SG_MAX_COPY_BATCH + 1];
+    sg_copy c[SG_MAX_COPY_BATCH];
+};
+
+__global__ __launch_bounds__(kNeuronBlock) void copy_u32_kernel(CopyBatch b) {
+    int j = 0;
+    while (j + 1 < b.n && (int)blockIdx.x >= b.first[j + 1]) ++j;
+    const uint32_t *src = static_cast<const uint32_t *>(b.c[j].src);
+    uint32_t *dst = static_cast<uint32_t *>(b.c[j].dst);
+    const long n = b.c[j].n;
+    const long stride = (long)(b.first[j + 1] - b.first[j]) * blockDim.x;
+    const long i0 =
+        (long)(blockIdx.x - b.first[j]) * blockDim.x + threadIdx.x;
     long done = 0;
-    if (vec) {
+    if (((uintptr_t)src | (uintptr_t)dst) % 16 == 0) {
         const long n4 = n / 4;
         for (long i = i0; i < n4; i += stride)
             ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
@@ -572,19 +584,37 @@ extern "C" int sg_hip_copy32(const void *src, void *dst, long n,
     return hipGetLastError();
 }
 
+extern "C" int sg_hip_copies_u32(const sg_copy *copies, int n, void *stream) {
+    for (int s0 = 0; s0 < n; s0 += SG_MAX_COPY_BATCH) {
+        CopyBatch b;
+        b.n = 0;
+        int blocks = 0;
+        for (int j = s0; j < n && j < s0 + SG_MAX_COPY_BATCH; ++j) {
+            const sg_copy &c = copies[j];
+            if (c.n <= 0) continue;
+            const uintptr_t at = (uintptr_t)c.src | (uintptr_t)c.dst;
+            if (at % 4 != 0) return (int)hipErrorInvalidValue;
+            const long units = at % 16 == 0 ? c.n / 4 + 3 : c.n;
+            b.c[b.n] = c;
+            b.first[b.n] = blocks;
+            blocks += (int)std::min<long>((units + kNeuronBlock - 1) /
+                                          kNeuronBlock, 1024L);
+            ++b.n;
+        }
+        if (b.n == 0) continue;
+        b.first[b.n] = blocks;
+        hipLaunchKernelGGL(copy_u32_kernel, dim3(blocks), dim3(kNeuronBlock),
+                           0, (hipStream_t)stream, b);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+
 extern "C" int sg_hip_copy_u32(const void *src, void *dst, long n,
                                void *stream) {
-    if (n <= 0) return 0;
-    if (((uintptr_t)src | (uintptr_t)dst) % 4 != 0)
-        return (int)hipErrorInvalidValue;
-    const int vec = ((uintptr_t)src | (uintptr_t)dst) % 16 == 0;
-    const long units = vec ? n / 4 + 3 : n;
-    const int blocks = (int)std::min<long>((units + kNeuronBlock - 1) /
-                                           kNeuronBlock, 1024L);
-    hipLaunchKernelGGL(copy_u32_kernel, dim3(blocks), dim3(kNeuronBlock), 0,
-                       (hipStream_t)stream, (const uint32_t *)src,
-                       (uint32_t *)dst, n, vec);
-    return hipGetLastError();
+    const sg_copy c = {src, dst, n};
+    return sg_hip_copies_u32(&c, 1, stream);
 }
 
 extern "C" int sg_hip_device_count(void) {

@@ -1499,22 +1499,35 @@ void Runner::updates() {
 bool Runner::output_issue(long it) {
     if (!(it % env_rate_ == 0 && !suppress_ && !out_keys_.empty()))
         return false;
+    // every copy of a stream in one launch, with the event of one of them
+    struct Group {
+        std::vector<sg_copy> copies;
+        std::vector<Res> reads;
+        HostBuf *last = nullptr;
+    };
+    std::map<int, Group> groups;
     for (auto &kv : out_keys_) {
         LayerState *ls = kv.first;
+        Group &g = groups[main_of(ls)];
         for (auto &k : kv.second) {
             HostBuf &b = *out_bufs_.at({ls, k});
             const void *src = k == "output" ? ls->output.dev
                             : k == "input" ? ls->input.dev
                             : ls->var(k).dev;
-            const Res r = k == "output" ? res(RES_OUT, ls)
-                        : k == "input" ? res(RES_IN, ls)
-                        : res(RES_STATE, ls);
-            hipStream_t s = sched().begin(main_of(ls), {r}, {});
-            check_hip(sg_hip_copy_u32(src, b.dp, ls->layer->size, s),
-                      "output copy");
-            sched().end();
-            b.record(s);
+            g.reads.push_back(k == "output" ? res(RES_OUT, ls)
+                              : k == "input" ? res(RES_IN, ls)
+                              : res(RES_STATE, ls));
+            g.copies.push_back(sg_copy{src, b.dp, ls->layer->size});
+            g.last = &b;
         }
+    }
+    for (auto &kv : groups) {
+        Group &g = kv.second;
+        hipStream_t s = sched().begin(kv.first, g.reads, {});
+        check_hip(sg_hip_copies_u32(g.copies.data(), (int)g.copies.size(), s),
+                  "output copies");
+        sched().end();
+        g.last->record(s);
     }
     return true;
 }

@@ -182,6 +182,12 @@ int sg_hip_iz_neurons(const sg_iz_layer *layers, int n, void *) {
 }
 // the engine's environment I/O: copied, so that the sanitizer sees both
 // ranges
+int sg_hip_copies_u32(const sg_copy *c, int n, void *) {
+    ++g_launches;
+    for (int i = 0; i < n; ++i)
+        if (c[i].n > 0) memmove(c[i].dst, c[i].src, (size_t)c[i].n * 4);
+    return 0;
+}
 int sg_hip_copy_u32(const void *src, void *dst, long n, void *) {
     ++g_launches;
     if (n > 0) memmove(dst, src, (size_t)n * 4);
