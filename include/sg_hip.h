@@ -341,9 +341,9 @@ int sg_hip_gol_steps(const uint32_t *words_in, uint32_t *words_out,
 /* A long run of a kernel of 0s and 1s (the same words as `steps` steps of
  * sg_hip_gol_steps; a positive multiple of 16): the words are turned into
  * bit planes in `planes` (scratch of sg_hip_gol_planes_bytes bytes, aligned
- * to 16; 0 bytes: other kernels, not taken here), stepped there, and turned
- * back into words_out, which may be words_in.  `launches` (or NULL) receives
- * the number of kernels launched. */
+ * to 16; 0 bytes: not taken here -- other kernels, or more than 262140 rows),
+ * stepped there, and turned back into words_out, which may be words_in.
+ * `launches` (or NULL) receives the number of kernels launched. */
 long sg_hip_gol_planes_bytes(const float *kernel9, int rows, int cols);
 int sg_hip_gol_planes(const uint32_t *words_in, uint32_t *words_out,
                       uint32_t *planes, int rows, int cols, int wrap,

@@ -1009,7 +1009,9 @@ static int plane_steps(int rows, int cols) {
 
 extern "C" long sg_hip_gol_planes_bytes(const float *k, int rows, int cols) {
     uint32_t wmask;
-    if (rows <= 0 || cols <= 0 || !bit_weights(k, wmask)) return 0;
+    // the turns' grids take four rows a block row, 65535 of those
+    if (rows <= 0 || rows > 4 * 65535 || cols <= 0 || !bit_weights(k, wmask))
+        return 0;
     return (long)sg::kGolRing * ((cols + 31) / 32) * sg::gol_pitch(rows) * 4;
 }
 
@@ -1020,7 +1022,8 @@ extern "C" int sg_hip_gol_planes(const uint32_t *words_in,
                                  int steps, int *launches, void *stream) {
     using namespace sg;
     uint32_t wmask, surv, birth;
-    if (steps < 1 || steps % 16 != 0 || !bit_weights(k, wmask))
+    if (steps < 1 || steps % 16 != 0 || rows > 4 * 65535 ||
+        !bit_weights(k, wmask))
         return (int)hipErrorInvalidValue;
     if (rows <= 0 || cols <= 0) return 0;
     rule_flags(smin, smax, bmin, bmax, surv, birth);

@@ -83,6 +83,11 @@ def test_planes_match_words(rows, cols, wrap, steps, rule):
                                   cols, wrap, kernel, *rule, 8, stream) == 0
         a, b = b, a
     assert torch.equal(a, got)
+    # refused before any launch: too tall a board, another kernel
+    assert L.sg_hip_gol_planes_bytes(kernel, 4 * 65535 + 1, 20) == 0
+    assert L.sg_hip_gol_planes(
+        words.data_ptr(), got.data_ptr(), planes.data_ptr(), 4 * 65535 + 1,
+        1, wrap, kernel, *rule, 16, None, stream) != 0
     other = (ctypes.c_float * 9)(1, 2, 1, 1, 0, 1, 1, 1, 1)
     assert L.sg_hip_gol_planes_bytes(other, rows, cols) == 0
     assert L.sg_hip_gol_planes(
