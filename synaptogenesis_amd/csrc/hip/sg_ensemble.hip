@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -36,6 +37,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+constexpr size_t kPageable = 1 << 18;
 constexpr int kTileRows = 16;   // BF16 row tile
 constexpr int kTileCols = 32;   // BF16 column tile
 constexpr int kGroupRows = 4;   // FP32 rows per wavefront
@@ -415,7 +417,8 @@ struct sg_ens {
     int persist_blocks = 0;
     int persist_captured = 0;
     // host reads: single reads since the state last changed, the whole state
-    // in pinned memory once they add up, and whether it is current
+    // on the host once they add up (pinned past kPageable floats: below that
+    // a pageable copy costs no more), and whether it is current
     std::mutex read_lock;
     int reads = 0;
     float *mirror = nullptr;
@@ -784,7 +787,8 @@ void sg_ens_destroy(sg_ens *e) {
     if (e->d_layers) (void)hipFree(e->d_layers);
     if (e->d_items) (void)hipFree(e->d_items);
     if (e->d_queue) (void)hipFree(e->d_queue);
-    if (e->mirror) (void)hipHostFree(e->mirror);
+    if (e->mirror && e->state_floats <= kPageable) free(e->mirror);
+    else if (e->mirror) (void)hipHostFree(e->mirror);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -1011,9 +1015,13 @@ int sg_ens_read_state(sg_ens *e, int inst, int layer, float *host) {
                                 hipMemcpyDeviceToHost), "read state");
             return 0;
         }
-        if (!e->mirror)
+        if (!e->mirror && e->state_floats <= kPageable) {
+            e->mirror = (float *)malloc(e->state_floats * 4);
+            if (!e->mirror) return fail("read states: no memory");
+        } else if (!e->mirror) {
             ENS_CHECK(hipHostMalloc((void **)&e->mirror, e->state_floats * 4,
                                     hipHostMallocDefault), "hipHostMalloc");
+        }
         ENS_CHECK(hipMemcpyAsync(e->mirror, e->d_state, e->state_floats * 4,
                                  hipMemcpyDeviceToHost, e->stream),
                   "read states");
