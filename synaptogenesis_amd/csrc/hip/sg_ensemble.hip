@@ -1009,18 +1009,22 @@ int sg_ens_read_state(sg_ens *e, int inst, int layer, float *host) {
     if (!e->mirrored) {
         ENS_CHECK(hipDeviceSynchronize(), "sync");
         const double whole = 30e-6 + e->state_floats * 4 / 45e9;
-        if (e->captured || e->reads * 24e-6 < whole) {
+        const bool one = e->captured || e->reads * 24e-6 < whole;
+        if (!one && !e->mirror) {
+            if (e->state_floats <= kPageable)
+                e->mirror = (float *)malloc(e->state_floats * 4);
+            else if (hipHostMalloc((void **)&e->mirror, e->state_floats * 4,
+                                   hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();    // not the next call's error
+                e->mirror = nullptr;
+            }
+        }
+        // without memory for the whole state every read is its own copy
+        if (one || !e->mirror) {
             ++e->reads;
             ENS_CHECK(hipMemcpy(host, e->d_state + off, bytes,
                                 hipMemcpyDeviceToHost), "read state");
             return 0;
-        }
-        if (!e->mirror && e->state_floats <= kPageable) {
-            e->mirror = (float *)malloc(e->state_floats * 4);
-            if (!e->mirror) return fail("read states: no memory");
-        } else if (!e->mirror) {
-            ENS_CHECK(hipHostMalloc((void **)&e->mirror, e->state_floats * 4,
-                                    hipHostMallocDefault), "hipHostMalloc");
         }
         ENS_CHECK(hipMemcpyAsync(e->mirror, e->d_state, e->state_floats * 4,
                                  hipMemcpyDeviceToHost, e->stream),
