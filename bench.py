@@ -179,9 +179,11 @@ def _workloads():
                      step_bytes=4228000, cpu_steps=300, detail="",
                      data="synthetic (Philox-seeded weights U[0,0.5); "
                           "device-drawn N(5,2) input into L1)"),
-        # launch_bytes: one launch reads and writes every word once, for
-        # the several steps it takes (8 on both boards; "game of life
-        # launches" in the report)
+        # launch_bytes: one launch on words reads and writes every word
+        # once, for the several steps it takes (8 on both boards).  Long
+        # runs take most steps as bit planes ("game of life launches" in
+        # the report counts them too); the kernel timed here is that of the
+        # run's last steps.
         "gol1024": dict(make=lambda: workloads.gol(1024), kernel="gol_step",
                         label="gol_step (8 steps per launch on bit-packed "
                               "rows: 3x3 count + rule + shift)",
