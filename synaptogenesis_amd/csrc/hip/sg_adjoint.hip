@@ -92,12 +92,14 @@ __device__ __forceinline__ float act_grad_fast(float u, int mode, float slope) {
 }
 
 // The same with one Newton step on the reciprocal (below 1 ulp again), for
-// the sizes whose passes divided exactly before they shared this scan.
+// the sizes whose passes divided exactly before they shared this scan.  No
+// step from a d past FP32: its reciprocal is 0 there as the division's was,
+// and the step would be infinity times 0.
 __device__ __forceinline__ float act_grad_newton(float u, int mode,
                                                  float slope) {
     const float d = 1.0f + slope * fabsf(u);
     const float r0 = __builtin_amdgcn_rcpf(d);
-    const float r = fmaf(r0, fmaf(-d, r0, 1.0f), r0);
+    const float r = d < INFINITY ? fmaf(r0, fmaf(-d, r0, 1.0f), r0) : r0;
     const float g = r * r;
     return mode == SG_SNN_SPIKE ? g : 0.5f * slope * g;
 }

@@ -36,3 +36,31 @@ def test_rate_gradients(batch, steps, n_in, n_hid, n_out, ck):
         return
     _close(g1, d1, 1e-4)
     _close(g2, d2, 1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_hid", [255, 256, 257])
+def test_potentials_past_the_derivative(n_hid):
+    """Potentials of 2e37 to 2e38, finite, whose 1 + slope |u| is not: the
+    surrogate derivative there is 0 (in FP64 below 1e-75), in the hidden
+    layer (one unit, from one step on) and in the output layer (one output,
+    whose large weight comes from a unit that spikes at the first step).
+    Spike mode: the bounds of test_gpu_snn.py."""
+    print("case snn potentials past the derivative", n_hid, flush=True)
+    cfg, x, w1, w2, labels = _case(adj.SPIKE, batch=3, steps=8, n_in=24,
+                                   n_hid=n_hid, n_out=5, ck=4)
+    x[:, :, 0] = 0
+    x[2, 1, 0] = 1
+    w1[7, 0] = 1e38             # row 1 of the batch, from step 2
+    x[0, :, 1] = 1
+    w1[9, 1] = 8
+    w2[:, 9] = 0
+    w2[2, 9] = 3e37             # every row, from step 0
+    w1, w2 = (w.bfloat16().float() for w in (w1, w2))
+    loss, counts, g1, g2 = _run(cfg, x, w1, w2, labels)
+    _, _, oloss, ocounts, d1, d2 = _oracle(cfg, x, w1, w2, labels)
+    assert np.array_equal(counts, ocounts)
+    assert abs(loss - oloss) <= 1e-5 * abs(oloss)
+    assert np.isfinite(g1).all() and np.isfinite(g2).all()
+    _close(g1, d1, 1e-3)
+    _close(g2, d2, 1e-3)
