@@ -45,6 +45,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -671,10 +672,12 @@ __global__ __launch_bounds__(256) void gemm_dw1_dma(
     const int hw = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
     const int lg = (nb % 8 == 0) ? (hw % 8) * (nb / 8) + hw / 8 : hw;
     const int bx = lg % nx, by = (lg / nx) % ny, bz = lg / (nx * ny);
-    if (dw2 && bz == (int)gridDim.z - 1) {
-        // the last z slice sums dW2 (dw2_reduce's work) beside the product
+    if (dw2 && bz >= kTnSplit) {
+        // the z slices past the product's sum dW2 (dw2_reduce's work)
+        // beside it
         const int ng = (O * H + 63) / 64;
-        for (int g = bx + nx * by; g < ng; g += nx * ny)
+        for (int g = bx + nx * (by + ny * (bz - kTnSplit)); g < ng;
+             g += nx * ny * ((int)gridDim.z - kTnSplit))
             dw2_reduce_block(part2, dw2, chunks2, H, O, scale, g);
         return;
     }
@@ -1585,6 +1588,21 @@ size_t dw2_slots(const sg_snn_cfg &c) {
         : ((size_t)c.checkpoint * c.batch + kDw2Rows - 1) / kDw2Rows;
 }
 
+// z slices of the dW1 product's launch that sum dW2, `xy` blocks each.  One,
+// whose blocks walk all of dW2's groups of 64 outputs, until a block's walk
+// is about as long as the product beside it (2048 slots of 14 ns); then a
+// slice for every 2048, as far as all of the launch's blocks stay resident,
+// two a CU (72 KB of LDS).  Forward and backward, one
+// slice against one a group: batch 4096, 64 -> 100 -> 10, 25 steps, 16 groups
+// on one block 1157 / 503 us; batch 1024, 128 -> 128 -> 10 261 / 244 us; batch
+// 512, 784 -> 1024 -> 10, past the resident blocks 342 / 396 us.
+unsigned dw2_slices(int xy, int outputs, int slots) {
+    const int groups = (outputs + 63) / 64, walks = (groups + xy - 1) / xy;
+    const long wanted = ((long)walks * slots + 2047) / 2048;
+    const long room = 512 / xy - kTnSplit;
+    return (unsigned)std::max(1L, std::min({wanted, room, (long)walks}));
+}
+
 Layout layout(const sg_snn_cfg &c) {
     const size_t B = c.batch, H = c.n_hid, O = c.n_out, ck = c.checkpoint;
     const size_t slots = (size_t)c.steps / ck + 1;
@@ -1861,8 +1879,9 @@ static int backward(const sg_snn_cfg *cfg, const uint16_t *x,
     const int per = ((MT + kTnSplit - 1) / kTnSplit + kDr - 1) / kDr * kDr;
     const dim3 dgrid((c.n_in + kDk - 1) / kDk, (H + kDh - 1) / kDh, kTnSplit);
     if (H % 4 == 0) {
-        // one more z slice of blocks sums dW2
-        const dim3 g2(dgrid.x, dgrid.y, kTnSplit + 1);
+        // and z slices of blocks that sum dW2
+        const dim3 g2(dgrid.x, dgrid.y,
+                      kTnSplit + dw2_slices(dgrid.x * dgrid.y, O * H, chunks));
         hipLaunchKernelGGL(gemm_dw1_dma, g2, dim3(256), 0, s, lam, xp, part1,
                            MT, H, c.n_in, per, gp, part2, dw2, chunks, O, grad);
     } else {

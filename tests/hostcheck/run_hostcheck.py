@@ -88,6 +88,15 @@ def main():
         assert got == launches, (n, got, launches)
     net.free()
     print("%-16s ok" % "gol grouping", flush=True)
+    # Beside other layers or callbacks an interrupt ends the run within the
+    # steps of one launch on words.
+    sess = harness.Session(
+        netdefs.gol_beside_relay(lib.interrupt_engine, 40), lib)
+    rep = sess.run(3000)
+    assert rep.get("interrupted") == "true", rep
+    assert 40 < int(rep.get("iterations")) <= 48, rep.get("iterations")
+    sess.free()
+    print("%-16s ok" % "gol interrupt", flush=True)
     stub = ctypes.CDLL(LIB)
     stub.hip_stub_bad_waits.restype = ctypes.c_long
     bad = stub.hip_stub_bad_waits()

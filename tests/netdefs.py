@@ -813,6 +813,23 @@ def all_cases():
         [dendrites(), second_order(), second_order_conv(), random_proj()]
 
 
+def gol_beside_relay(interrupt, at, rows=20, cols=24, steps=3000,
+                     name="gol_beside_relay"):
+    """A game-of-life board that nothing reads beside a relay layer with
+    per-step input; the input callback of step `at` calls `interrupt`."""
+    case = gol(name, rows, cols, steps, 119)
+    case.net["structures"][0]["layers"].append(layer("in", "relay", 4, 4))
+
+    def feed(t):
+        if t == at:
+            interrupt()
+        return np.full(16, t, np.float32)
+
+    case.inputs = {("gol", "in"): feed}
+    case.capture = [("gol", "in", "output")]
+    return case
+
+
 # -- the benchmark configurations at their stated size and length ------------
 # Their fixtures keep one record per step (harness.long_record: a 64-bit
 # digest of each captured array and the layer's spike count), written by

@@ -73,3 +73,50 @@ def test_reads_follow_every_change():
         assert np.array_equal(every(e)[1], new)
     e.close()
     f.close()
+
+
+@pytest.mark.gpu
+def test_reads_after_a_callers_graph():
+    """Runs recorded into a caller's graph change the state at every replay,
+    unseen by the ensemble: however many states were read before, each read
+    shows the state as it is."""
+    import torch
+    widths = [[40, 70, 33], [5, 64, 100], [17, 3, 9]]
+    e = RateEnsemble(widths, "bf16", leak=0.5)
+    f = RateEnsemble(widths, "bf16", leak=0.5)
+
+    def every(a):
+        return [a.state(i, k) for i in range(3) for k in range(3)]
+
+    for _ in range(3):
+        every(e)                # the whole state on the host
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=stream):
+        e.run(2, graph=False,
+              stream=torch.cuda.current_stream().cuda_stream)
+    for replay in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        f.run(2, graph=False)
+        for _ in range(3):
+            for x, y in zip(every(e), every(f)):
+                assert np.array_equal(x, y)
+        if replay == 1:         # the program's own steps in between
+            e.run(2)
+            f.run(2)
+    e.close()
+    f.close()
+
+
+@pytest.mark.gpu
+def test_read_without_a_buffer_is_refused():
+    """A null buffer is an error, also where the read would be served from
+    the host copy of the whole state."""
+    e = RateEnsemble([[40, 70, 33]], "bf16")
+    for _ in range(20):
+        e.state(0, 1)
+    assert e.lib.sg_ens_read_state(e.handle, 0, 1, None) != 0
+    assert e.state(0, 1).shape == (70,)
+    e.close()

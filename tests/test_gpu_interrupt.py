@@ -58,3 +58,26 @@ def test_interrupt_engine_from_another_thread_then_resume(gpu_lib):
             assert a.tobytes() == b.tobytes(), (k, t)
     for k in wfins:
         assert fins[k].tobytes() == wfins[k].tobytes(), k
+
+
+@pytest.mark.gpu
+def test_interrupt_from_a_callback_beside_a_board(gpu_lib):
+    """A board takes several steps a launch (eight at most beside other
+    layers), and an interrupt ends the run where the last of them ends: the
+    callbacks go on for no more than those."""
+    print("case interrupt from a callback beside a board", flush=True)
+    at = 40
+    sess = harness.Session(
+        netdefs.gol_beside_relay(gpu_lib.interrupt_engine, at), gpu_lib)
+    rep = sess.run(3000)
+    done = int(rep.get("iterations"))
+    assert rep.get("interrupted") == "true"
+    assert at < done <= at + 8
+    fed, fins = sess.captures[("gol", "in", "output")], sess.finals()
+    sess.free()
+    assert len(fed) == done
+    whole = harness.Session(netdefs.gol_beside_relay(None, -1), gpu_lib)
+    whole.run(done)
+    key = ("neuron", "gol", "board", "output")
+    assert whole.finals()[key].tobytes() == fins[key].tobytes()
+    whole.free()

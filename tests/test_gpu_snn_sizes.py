@@ -18,7 +18,10 @@ from test_gpu_snn import _case, _close, _oracle, _run
 SIZES = [(1, 12, 8, 1, 1, 4), (2, 16, 40, 63, 10, 16),
          (3, 32, 113, 255, 16, 16), (4, 12, 127, 257, 2, 3),
          (5, 20, 129, 260, 10, 10), (2, 12, 784, 500, 10, 6),
-         (130, 12, 16, 513, 3, 12)]
+         (130, 12, 16, 513, 3, 12),
+         # dW2 summed by 1, 2 and 6 slices of blocks beside dW1's product
+         (409, 6, 8, 64, 5, 3), (410, 6, 8, 64, 5, 3),
+         (700, 4, 120, 128, 16, 2)]
 
 
 @pytest.mark.gpu
