@@ -696,18 +696,26 @@ class Runner {
     std::map<LayerState *, uint32_t *> gol_home_;
     // game-of-life layers that nothing else reads (their only outgoing
     // connection is the self-connection): stepped up to
-    // sg_hip_gol_max_steps steps per launch in eager runs; gol_ahead_ counts the steps an earlier launch already
-    // took beyond the current one, gol_rem_ the steps left in the run from
-    // the current one (1 while steps are captured into graphs)
+    // sg_hip_gol_max_steps steps per launch in eager runs; gol_ahead_ counts
+    // the steps an earlier launch already took beyond the current one,
+    // gol_rem_ the steps left in the run from the current one (1 while steps
+    // are captured into graphs)
     std::set<LayerState *> gol_multi_;
     std::map<LayerState *, int> gol_ahead_;
     long gol_rem_ = 1;
     long gol_launches_ = 0;
     // With more than this many steps left a layer of a 0/1 kernel takes them
-    // as bit planes, at most so many at once (an interrupt waits for them):
-    // turning a 1024 x 1024 board into planes and back costs about what 16
-    // steps on words do, and the planes halve the rest.
+    // as bit planes, at most so many at once: turning a board into planes
+    // and back costs what 11 to 26 steps on words do, and a step on planes a
+    // third to a half of one on words (128 steps: 64 x 64 37 us for 83, 1024 x
+    // 1024 56 for 116, 16384 x 16384 5.4 ms for 8.3).  Only where all layers
+    // are such boards and no module runs: an interrupt waits for the steps
+    // taken ahead, and so would other layers and their callbacks, each of
+    // those steps at their own pace.
     static constexpr long kGolPlanesFrom = 128, kGolPlanesMost = 4096;
+    bool gol_alone() const {
+        return modules_.empty() && gol_multi_.size() == st_->layers().size();
+    }
     uint32_t *gol_planes_of(LayerState *ls, const float *k9);
     bool gol_pending() const {
         for (const auto &kv : gol_ahead_)
@@ -1275,7 +1283,7 @@ void Runner::update_neurons(const std::vector<LayerState *> &lss, int sidx,
                                              : iterations_ != 0 && k == gol_rem_;
                     uint32_t *spare = C_->gol_spare.at(ls);
                     uint32_t *planes = nullptr;
-                    if (gol_multi_.count(ls) && gol_rem_ > kGolPlanesFrom)
+                    if (gol_alone() && gol_rem_ > kGolPlanesFrom)
                         planes = gol_planes_of(ls, k9);
                     if (planes) {
                         // all but the last steps, which write the input
