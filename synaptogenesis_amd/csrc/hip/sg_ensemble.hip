@@ -1001,6 +1001,7 @@ int sg_ens_autotune(sg_ens *e, int steps, int *row_tiles, int *k_split,
 // (2 x 256 of them: 13 ms) pays at most twice the whole copy.
 int sg_ens_read_state(sg_ens *e, int inst, int layer, float *host) {
     if (check_inst(e, inst, layer, 0)) return 1;
+    if (!host) return fail("read state: null buffer");
     std::lock_guard<std::mutex> lock(e->read_lock);
     const long off = layer == 0 ? e->x0_off[inst]
                    : layer == 1 ? e->h1_off[e->parity][inst]
