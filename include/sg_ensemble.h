@@ -56,12 +56,13 @@ sg_ens *sg_ens_create(int n, const int *widths, int precision, float leak,
                       int rectify, uint64_t seed, uint32_t workload);
 void sg_ens_destroy(sg_ens *e);
 
-/* Launch shape: row_tiles 16-row tiles per block, each split over
- * k_split wavefronts along the fan-in (BF16: row_tiles * k_split in
- * {1,2,4,8,16} wavefronts; FP32: k_split must be 1, row_tiles 4-row
- * groups).  Changing it drops any captured graph.  It first waits for
- * every run still pending (on the ensemble's stream and on the stream of
- * the last sg_ens_run), whose kernels read the work list it rewrites. */
+/* Launch shape (by the ensemble's size where none is set): row_tiles 16-row
+ * tiles per block, each split over k_split wavefronts along the fan-in
+ * (BF16: row_tiles * k_split in {1,2,4,8,16} wavefronts; FP32: k_split must
+ * be 1, row_tiles 4-row groups).  Changing it drops any captured graph.  It
+ * first waits for every run still pending (on the ensemble's stream and on
+ * the stream of the last sg_ens_run), whose kernels read the work list it
+ * rewrites. */
 int sg_ens_set_tile(sg_ens *e, int row_tiles, int k_split);
 int sg_ens_get_tile(const sg_ens *e, int *row_tiles, int *k_split);
 
@@ -104,7 +105,13 @@ int sg_ens_time_steps(sg_ens *e, int steps, float *avg_ms);
 
 /* Host copies (synchronous).  layer 0 = x0, 1 = h1, 2 = h2 (current
  * values, `width` floats).  Weights: layer 1 or 2, row-major
- * [fan_out][fan_in] FP32 values as the kernels use them. */
+ * [fan_out][fan_in] FP32 values as the kernels use them.
+ * After some state reads with no change in between, the whole state is
+ * copied to the host (memory of its size, kept until sg_ens_destroy) and
+ * further reads are served from there, without a device synchronisation,
+ * until the next run, write, timing or tuning of this ensemble.  Once a run
+ * has been recorded into a caller's graph, whose replays the ensemble does
+ * not see, every read is a copy from the device. */
 int sg_ens_read_state(sg_ens *e, int inst, int layer, float *host);
 int sg_ens_write_state(sg_ens *e, int inst, int layer, const float *host);
 int sg_ens_read_weights(sg_ens *e, int inst, int layer, float *host);

@@ -567,17 +567,16 @@ hipError_t launch_persistent(sg_ens *e, int steps, int parity,
 struct Change {
     sg_ens *e;
     Change(sg_ens *e_, hipStream_t s) : e(e_) {
-        drop();
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (s && hipStreamIsCapturing(s, &st) == hipSuccess &&
-            st != hipStreamCaptureStatusNone)
-            e->captured = true;
+        drop(s && hipStreamIsCapturing(s, &st) == hipSuccess &&
+             st != hipStreamCaptureStatusNone);
     }
-    ~Change() { drop(); }
-    void drop() {
+    ~Change() { drop(false); }
+    void drop(bool recorded) {
         std::lock_guard<std::mutex> lock(e->read_lock);
         e->reads = 0;
         e->mirrored = false;
+        if (recorded) e->captured = true;
     }
 };
 
