@@ -726,7 +726,7 @@ class Runner {
     bool any_dendrites_ = false, any_second_order_ = false;
 
     std::map<const Structure *, int> main_, side_;
-    int nstreams_ = 1;
+    int nstreams_ = 1, structure_streams_ = 1;  // in all; structures' own
     bool any_split_ = false;
 };
 
@@ -998,6 +998,7 @@ void Runner::setup_streams() {
     for (size_t si = 0; si < structs.size(); ++si)
         main_[structs[si].get()] = per_structure ? next++ : 0;
     if (next == 0) next = 1;
+    structure_streams_ = next;
     for (size_t si = 0; si < structs.size(); ++si) {
         const Structure *s = structs[si].get();
         bool any_base = false, any_other = false;
@@ -1725,15 +1726,15 @@ Props *Runner::run() {
 
     // With "step graphs": "true", runs without environment I/O capture their
     // steady-state steps (from the second on, all but the last) into HIP
-    // graphs of `block` steps -- when at most two streams take part (one
-    // structure and its activator stream): a capture over three streams
-    // (two structures) ended the process with a segmentation fault on the
+    // graphs of `block` steps -- on one structure's stream, alone or with its
+    // activator stream: a capture over the streams of two structures (three
+    // streams in all) ended the process with a segmentation fault on the
     // GPU host once, cause not found, so such runs stay eager.  Off by
     // default: on the benchmark networks the GPU, not the host's launches,
     // bounds the step (the same step time with and without graphs), and a
     // capture costs milliseconds.
     const bool graphs = modules_.empty() && !kt_.on && !any_second_order_ &&
-                        nstreams_ <= 2 &&
+                        structure_streams_ == 1 && nstreams_ <= 2 &&
                         args_.get_bool("step graphs", false) &&
                         iterations_ > 0;
     int block = std::max(2, args_.get_int("graph steps", 8));

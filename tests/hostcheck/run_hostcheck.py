@@ -28,6 +28,7 @@ from synaptogenesis_amd import syngen, workloads  # noqa: E402
 import bench  # noqa: E402
 import harness  # noqa: E402
 import netdefs  # noqa: E402
+import test_gpu_streams  # noqa: E402
 
 LIB = os.path.join(HERE, "_build", "libsyngen_hostcheck.so")
 
@@ -64,6 +65,10 @@ def main():
                       {"compact records": "false"}):
             rep = sess.run(11, extra)
             assert rep.get("iterations") == "11", (case.name, extra)
+            # no capture over the streams of several structures
+            if (len(case.net["structures"]) > 1 and
+                    "structure streams" not in extra):
+                assert rep.get("step graphs") == "0", (case.name, extra)
         sess.finals()
         sess.free()
         print("%-16s ok" % case.name, flush=True)
@@ -88,6 +93,16 @@ def main():
         assert got == launches, (n, got, launches)
     net.free()
     print("%-16s ok" % "gol grouping", flush=True)
+    # Two structures: steps are captured with both on one stream only.
+    for extra, captured in (({}, False),
+                            ({"concurrent activators": "true"}, False),
+                            ({"structure streams": "false"}, True)):
+        net = bench.build(lib, test_gpu_streams._two_structures())
+        _, rep = bench.run(net, 40, dict(extra, **{"step graphs": "true"}))
+        assert (int(rep.get("step graphs")) > 0) == captured, (
+            extra, rep.get("streams"), rep.get("step graphs"))
+        net.free()
+    print("%-16s ok" % "two structures", flush=True)
     # Beside other layers or callbacks an interrupt ends the run within the
     # steps of one launch on words.
     sess = harness.Session(

@@ -140,11 +140,13 @@ def _same(a, b):
 
 
 @pytest.mark.gpu
-def test_step_graphs_match_eager_steps(gpu_lib):
+@pytest.mark.parametrize("concurrent", ["false", "true"])
+def test_step_graphs_match_eager_steps(gpu_lib, concurrent):
     """Steady-state steps captured into HIP graphs (of 2, 8 and 16 steps,
-    the step counter of the random draws read on the device) leave every
-    array as the eager steps do."""
-    print("step graphs vs eager", flush=True)
+    the step counter of the random draws read on the device; one stream, or
+    a second one forked for the activators) leave every array as the eager
+    steps do."""
+    print("step graphs vs eager", concurrent, flush=True)
     wl = workloads.sheet(32, 40)
     eager, reps = _state_after(gpu_lib, wl, "sheet", ("E", "I"), ("EE",),
                                [STEPS], {"step graphs": "false"})
@@ -152,26 +154,35 @@ def test_step_graphs_match_eager_steps(gpu_lib):
     for block in ("2", "8", "16"):
         got, reps = _state_after(gpu_lib, wl, "sheet", ("E", "I"), ("EE",),
                                  [STEPS], {"step graphs": "true",
-                                           "graph steps": block})
+                                           "graph steps": block,
+                                           "concurrent activators":
+                                               concurrent})
         assert int(reps[0].get("step graphs")) > 0, block
+        assert reps[0].get("streams") == ("2" if concurrent == "true"
+                                          else "1")
         _same(eager, got)
     assert np.unpackbits(eager[("E", "output")].view(np.uint8)).sum() > 0
 
 
 @pytest.mark.gpu
-def test_runs_in_parts_match_one_run(gpu_lib):
+@pytest.mark.parametrize("concurrent", ["false", "true"])
+def test_runs_in_parts_match_one_run(gpu_lib, concurrent):
     """A deferred update crosses from one run into the next, and the
     random draws continue with the state's step count: 7 + 13 + 20 steps
     leave the arrays of one 40-step run, graphs or not."""
-    print("runs in parts", flush=True)
+    print("runs in parts", concurrent, flush=True)
     wl = workloads.sheet(32, 40)
     whole, _ = _state_after(gpu_lib, wl, "sheet", ("E", "I"), ("EE",),
                             [STEPS])
     parts, reps = _state_after(gpu_lib, wl, "sheet", ("E", "I"), ("EE",),
-                               [7, 13, 20], {"step graphs": "true"})
+                               [7, 13, 20], {"step graphs": "true",
+                                             "concurrent activators":
+                                                 concurrent})
+    assert all(int(r.get("step graphs")) > 0 for r in reps[1:])
     _same(whole, parts)
     eager, _ = _state_after(gpu_lib, wl, "sheet", ("E", "I"), ("EE",),
-                            [7, 13, 20])
+                            [7, 13, 20],
+                            {"concurrent activators": concurrent})
     _same(whole, eager)
 
 
@@ -238,10 +249,10 @@ def _two_state(lib, extra):
 
 @pytest.mark.gpu
 @pytest.mark.skip(reason="ended the test process with a segmentation fault "
-                  "on the GPU host (three streams; graph capture over more "
-                  "than two streams has been switched off since, cause not "
-                  "found); one stream per structure stays covered by the "
-                  "mixed_clusters golden case")
+                  "on the GPU host (three streams; graph capture over the "
+                  "streams of several structures has been switched off "
+                  "since, cause not found); one stream per structure stays "
+                  "covered by the mixed_clusters golden case")
 def test_structure_streams_match_one_stream(gpu_lib):
     """One stream per structure, ordered by the scheduler's events, leaves
     every array as everything on one stream does, with and without step
@@ -252,7 +263,11 @@ def test_structure_streams_match_one_stream(gpu_lib):
                                      "step graphs": "false"})
     assert rep1.get("streams") == "1"
     for graphs in ("false", "true"):
-        many, rep = _two_state(gpu_lib, {"step graphs": graphs})
-        assert int(rep.get("streams")) >= 3
-        _same(one, many)
+        for concurrent, streams in (("false", 2), ("true", 3)):
+            many, rep = _two_state(gpu_lib,
+                                   {"step graphs": graphs,
+                                    "concurrent activators": concurrent})
+            assert int(rep.get("streams")) >= streams
+            assert rep.get("step graphs") == "0"
+            _same(one, many)
     assert np.unpackbits(one[("C", "output")].view(np.uint8)).sum() > 0
