@@ -227,7 +227,8 @@ struct Cache : EngineCache {
     Sched sched;
     // second word buffer of each game-of-life layer on the fused step
     std::map<LayerState *, uint32_t *> gol_spare;
-    // bit planes of a game-of-life layer's long runs (null: no memory)
+    // bit planes of a game-of-life layer's long runs (null: no memory in
+    // the current run; the next one asks again)
     std::map<LayerState *, uint32_t *> gol_planes;
     // step counter that captured steps read their random draws' step from
     uint64_t *d_step = nullptr;
@@ -1676,6 +1677,8 @@ Props *Runner::run() {
     // Izhikevich records uploaded by this run.
     st_->to_device(args_.get_bool("compact records", true));
     C_ = &cache_of(*st_);
+    for (auto it = C_->gol_planes.begin(); it != C_->gol_planes.end();)
+        it = it->second ? std::next(it) : C_->gol_planes.erase(it);
     if (!C_->d_step) {
         check_hip(hipMalloc((void **)&C_->d_step, 8), "hipMalloc");
         check_hip(hipHostMalloc((void **)&C_->h_step, 8,

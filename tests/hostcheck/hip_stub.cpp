@@ -19,6 +19,7 @@ namespace {
 struct StubEvent { bool recorded = false; };
 struct StubStream { int capturing = 0; };
 std::atomic<long> g_bad_waits(0), g_waits(0), g_records(0), g_launches(0);
+std::atomic<size_t> g_refused(0);
 struct Report {
     ~Report() {
         if (getenv("HIP_STUB_REPORT"))
@@ -34,7 +35,12 @@ extern "C" {
 
 long hip_stub_bad_waits(void) { return g_bad_waits.load(); }
 
+// hipMalloc of exactly n bytes fails from here on (0: none does)
+void hip_stub_refuse(size_t n) { g_refused = n; }
+
 hipError_t hipMalloc(void **p, size_t n) {
+    *p = nullptr;
+    if (n && n == g_refused) return hipErrorOutOfMemory;
     *p = calloc(1, n ? n : 1);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -93,6 +93,18 @@ def main():
         assert got == launches, (n, got, launches)
     net.free()
     print("%-16s ok" % "gol grouping", flush=True)
+    # A board without room for its planes runs on words (8 steps a launch)
+    # and asks again with the next run (here all but 8 steps on planes, whose
+    # launches the stand-in does not count).
+    stub = ctypes.CDLL(LIB)
+    net = bench.build(lib, workloads.gol(64))
+    for refused, launches in ((6 * 64 * 64 + 64, 25), (0, 1), (0, 1)):
+        stub.hip_stub_refuse(ctypes.c_size_t(refused))
+        rep = net.run(None, {"iterations": "200"})
+        got = int(rep.get("game of life launches"))
+        assert got == launches, (refused, got, launches)
+    net.free()
+    print("%-16s ok" % "gol planes", flush=True)
     # Two structures: steps are captured with both on one stream only.
     for extra, captured in (({}, False),
                             ({"concurrent activators": "true"}, False),
@@ -112,7 +124,6 @@ def main():
     assert 40 < int(rep.get("iterations")) <= 48, rep.get("iterations")
     sess.free()
     print("%-16s ok" % "gol interrupt", flush=True)
-    stub = ctypes.CDLL(LIB)
     stub.hip_stub_bad_waits.restype = ctypes.c_long
     bad = stub.hip_stub_bad_waits()
     print("waits on unrecorded events: %d" % bad)
