@@ -80,6 +80,8 @@ SPARSE_TRAFFIC_SUMMARY = os.path.join(
     ROOT, "profiles", "iz_update_activate_sparse_sheet_traffic.txt")
 ENS_TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles",
                                    "ens_bf16_ensemble_traffic.txt")
+GOL_TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles",
+                                   "game_of_life_%d_planes_traffic.txt")
 
 
 def measured_traffic(path=TRAFFIC_SUMMARY, key="traffic_bytes_per_launch"):
@@ -179,27 +181,50 @@ def _workloads():
                      step_bytes=4228000, cpu_steps=300, detail="",
                      data="synthetic (Philox-seeded weights U[0,0.5); "
                           "device-drawn N(5,2) input into L1)"),
-        # launch_bytes: one launch on words reads and writes every word
-        # once, for the several steps it takes (8 on both boards).  Long
-        # runs take most steps as bit planes ("game of life launches" in
-        # the report counts them too); the kernel timed here is that of the
-        # run's last steps.
-        "gol1024": dict(make=lambda: workloads.gol(1024), kernel="gol_step",
-                        label="gol_step (8 steps per launch on bit-packed "
-                              "rows: 3x3 count + rule + shift)",
-                        launch_bytes=8 * 1024 * 1024,
-                        step_bytes=8 * 1024 * 1024, cpu_steps=40,
+        # the kernel, its bytes and its label depend on the run's length:
+        # gol_kernel()
+        "gol1024": dict(make=lambda: workloads.gol(1024), side=1024,
+                        planes_summary=GOL_TRAFFIC_SUMMARY % 1024,
+                        cpu_steps=40,
                         detail=" (3x3 convolutional, wrap, self excluded)",
                         data="synthetic (Philox Bernoulli(0.5) cells)"),
-        "gol16384": dict(make=lambda: workloads.gol(16384),
-                         kernel="gol_step",
-                         label="gol_step (8 steps per launch on bit-packed "
-                               "rows: 3x3 count + rule + shift)",
-                         launch_bytes=8 * 16384 * 16384,
-                         step_bytes=8 * 16384 * 16384, cpu_steps=1,
+        "gol16384": dict(make=lambda: workloads.gol(16384), side=16384,
+                         planes_summary=GOL_TRAFFIC_SUMMARY % 16384,
+                         cpu_steps=1,
                          detail=" (3x3 convolutional, wrap, self excluded)",
                          data="synthetic (Philox Bernoulli(0.5) cells)"),
     }
+
+
+def gol_kernel(spec, steps, timing, report):
+    """The roofline fields of a game-of-life run: of its time on bit planes
+    where it has one, else of its launches on words.  On planes a "launch" is
+    one timed call: the turn to planes (8 B a cell), plane launches of K steps
+    (each reads the newest plane and K old ones and writes K new ones, a bit
+    a cell) and the turn back.  On words a launch reads and writes every
+    word, and the run's last one the sums (4 B)."""
+    cells = spec["side"] ** 2
+    words = int(timing["gol_step launches"])
+    if "gol_planes ms" not in timing:
+        return dict(kernel="gol_step",
+                    label="gol_step (%d steps in %d launches on words)"
+                          % (steps, words),
+                    launch_bytes=cells * (8 + 4 / words),
+                    step_bytes=cells * (8 * words + 4) / steps)
+    calls = int(timing["gol_planes launches"])
+    total = int(report.get("game of life launches")) - words - 2 * calls
+    launches = total / calls
+    K = 16 if 16 * total < steps else 8
+    plane = measured_traffic(spec["planes_summary"])
+    turns = measured_traffic(spec["planes_summary"], "turn_traffic_bytes")
+    return dict(kernel="gol_planes",
+                label="gol_plane_kernel (%g launches of %d steps on bit "
+                      "planes, and the turns to and from them)"
+                      % (launches, K),
+                launch_bytes=cells * (16 + launches * (2 * K + 1) / 8),
+                step_bytes=cells * (2 * K + 1) / (8 * K),
+                traffic=launches * plane + turns if plane and turns else None,
+                traffic_summary=spec["planes_summary"])
 
 
 def build(lib, wl):
@@ -841,6 +866,8 @@ def main():
 
     ms_per_step = dt * 1000.0 / a.steps
     syn_per_s = wl["visits_per_step"] * a.steps / dt
+    if "side" in spec:
+        spec = dict(spec, **gol_kernel(spec, a.steps, timing, kreport))
     key = spec["kernel"]
     kernel_ms = float(timing[key + " ms"]) / float(timing[key + " launches"])
     launch_bytes = wl.get("launch_bytes", spec["launch_bytes"])
@@ -849,7 +876,8 @@ def main():
                for k, v in timing.items() if k.endswith(" ms")}
 
     tpath = spec.get("traffic_summary")
-    traffic = measured_traffic(tpath) if tpath else None
+    traffic = spec.get("traffic") or (measured_traffic(tpath) if tpath
+                                      else None)
     step_traffic = (measured_traffic(spec["step_traffic_summary"],
                                      "step_traffic_bytes")
                     if spec.get("step_traffic_summary") else None)

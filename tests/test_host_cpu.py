@@ -391,3 +391,28 @@ def test_randomized_convergent_moves_whole_fields(lib, wrap):
         corners.add((int(r[0]), int(c[0])))
     assert len(corners) > 40                 # drawn, not the regular grid
     network.free()
+
+
+def test_benchmark_names_the_game_of_life_kernel_it_times():
+    """bench.py's game-of-life roofline is that of the bit planes where the
+    run is spent there, with the planes' bytes: 992 of 1000 steps in 62
+    launches of 16 (33 planes of a bit a cell each) or 124 of 8 (17), and the
+    turns (16 B a cell); on words 8 B a cell a launch and the sums' 4 once."""
+    import bench
+    for side, launches, per, planes in ((1024, 62, 16, 33),
+                                        (16384, 124, 8, 17)):
+        spec = bench._workloads()["gol%d" % side]
+        got = bench.gol_kernel(
+            spec, 1000, {"gol_planes ms": "1", "gol_planes launches": "1",
+                         "gol_step ms": "1", "gol_step launches": "1"},
+            {"game of life launches": str(launches + 3)})
+        cells = side * side
+        assert got["kernel"] == "gol_planes"
+        assert "%d launches of %d steps" % (launches, per) in got["label"]
+        assert got["launch_bytes"] == cells * (16 + launches * planes / 8)
+        assert got["step_bytes"] == cells * planes / 8 / per
+        assert got["traffic"] > got["launch_bytes"]
+    got = bench.gol_kernel(spec, 16, {"gol_step ms": "1",
+                                      "gol_step launches": "2"}, {})
+    assert got["kernel"] == "gol_step"
+    assert got["launch_bytes"] == cells * 10
