@@ -80,8 +80,9 @@ typedef struct sg_conn {
      * layer's neuron kernel): skip packing it. */
     int plane_ready;
     /* Store each destination's sum itself into dst instead of aggregating
-     * it into the input; the neuron kernel then aggregates it into the
-     * layer's init-config value (sg_iz_layer.noise == 2). */
+     * it into the input: the neuron kernel aggregates it into the layer's
+     * init-config value (sg_iz_layer.noise == 2), or it is the first sum
+     * added to an input that would otherwise be cleared before. */
     int store_sum;
     /* SG_SPARSE: source index of visit k of slot s in device layout
      * (k_per_dest = the largest nonzero count), -1 past the slot's count
@@ -91,10 +92,10 @@ typedef struct sg_conn {
      * nonzero visits of its slots ({lo, hi} per tile); a tile's walk ends
      * at its hi, and visits below its lo need no check. */
     const int32_t *tile_counts;
-    /* The launch runs beside a long kernel on another stream: a base
-     * activator on the plane path then uses blocks of four wavefronts
-     * (they start as soon as a CU has four free wave slots) instead of
-     * sixteen. */
+    /* The launch runs beside a long kernel on another stream: where a base
+     * activator on the plane path has 64 destinations a block, the block then
+     * has four wavefronts (they start as soon as a CU has four free wave
+     * slots) instead of eight or sixteen. */
     int beside;
 } sg_conn;
 

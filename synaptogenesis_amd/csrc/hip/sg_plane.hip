@@ -252,29 +252,47 @@ __global__ __launch_bounds__(64) void plane_lane_kernel(sg_conn c,
     put_sum(c, slot_to_index(c, slot), sum);
 }
 
+// A lane per destination for up to 16 visits, and for more once the layer's
+// own wavefronts fill the GPU, the later the more visits there are: 25 visits
+// at 1024 tiles 9.3 us against 9.6 with eight wavefronts a tile, 49 at 1407
+// 14.8 against 13.8 and at 2025 15.9 against 18.3, 81 at 2500 28 against 26 and
+// at 2757 29 against 44.  SPARSE, whose indices a lane waits for: 30 visits at
+// 1563 tiles 11.5 against 10.2 and at 3125 18.5 against 22.8, 64 at 3125 30
+// against 25 and at 7813 48 against 49.
+static bool plane_lanes(int type, int count, int tiles) {
+    if (count <= 16) return true;
+    if (type == SG_SPARSE)
+        return count <= 64 && tiles >= (count <= 32 ? 2048 : 4096);
+    if (count <= 64) return tiles >= 1024 + 16 * (count > 25 ? count - 25 : 0);
+    return count <= 128 && tiles >= 2560;
+}
+
 // Which form (all give the same bits), by one sweep:
-// * a lane per destination for up to 16 visits, and for up to 64 once the
-//   layer's own wavefronts fill the GPU (1024 tiles): 5 x 5 on 512 x 512
-//   9.2 us against 37 with eight wavefronts a tile;
+// * a lane per destination (plane_lanes);
 // * 16 destinations a block while that gives every block a CU of its own
-//   (64 tiles): 15 x 15 on 64 x 64 6.9 us against 7.8;
+//   (64 tiles) and its chunk has more visits than one of sixteen wavefronts a
+//   tile: 21 x 21 on 64 x 64 11 us against 14, 11 x 11 9.3 against 7.8;
 // * beside a long kernel on another stream (sg_conn.beside), four
 //   wavefronts a tile: they start as soon as a CU has four free wave slots;
 // * sixteen wavefronts a tile up to two tiles a CU (15 x 15 on 128 x 128
 //   7.7 us against 10 with eight), eight beyond (on 256 x 256 17.9 against
-//   19.5).
+//   19.5), four of those blocks a CU; SPARSE also sixteen where a few tiles
+//   are left to a last round of eight (1032 tiles: 250 visits 34 us against 39,
+//   600 visits 85 against 105; 1563 tiles 45 against 41).
 template <int TYPE>
 static hipError_t launch_plane_t(const sg_conn &c, hipStream_t st) {
     const int count = cursor<TYPE>(c, 0).count;
     const int tiles = (c.num_dest + 63) / 64;
-    if (count <= 16 || (count <= 64 && tiles >= 1024)) {
+    if (plane_lanes(TYPE, count, tiles)) {
         hipLaunchKernelGGL(plane_lane_kernel<TYPE>, dim3(tiles), dim3(64), 0,
                            st, c, c.plane);
         return hipGetLastError();
     }
-    if (count > 64 && tiles <= 64) return launch_plane_w<TYPE, 16, 16>(c, st);
+    if (count > 128 && tiles <= 64) return launch_plane_w<TYPE, 16, 16>(c, st);
     if (c.beside) return launch_plane_w<TYPE, 64, 4>(c, st);
-    if (tiles <= 512) return launch_plane_w<TYPE, 64, 16>(c, st);
+    const bool few_left = TYPE == SG_SPARSE && count > 64 && tiles > 1024 &&
+                          tiles < 3072 && (tiles - 1) % 1024 < 256;
+    if (tiles <= 512 || few_left) return launch_plane_w<TYPE, 64, 16>(c, st);
     return launch_plane_w<TYPE, 64, 8>(c, st);
 }
 

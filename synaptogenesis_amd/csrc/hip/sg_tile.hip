@@ -42,11 +42,17 @@ static void launch_lane_type(const sg_conn &c, hipStream_t st) {
 
 // Which form of the base activator (all three give the same bits), from one
 // sweep of sizes:
-// * lanes alone once the layer's own wavefronts fill the GPU and the visits'
-//   sources have to be walked: convergent 5 x 5 on 256 x 256 (1024 tiles)
-//   6.1 us against 9.8, 15 x 15 on 360 x 360 (2025 tiles) 37.5 against 45
-//   (on 256 x 256: 35 against 24).  Fully connected layers need no walk and
-//   keep the tile kernel: 300 -> 131072 25 us against 47.
+// * lanes alone where a tile's visits would leave most of a block idle, up to
+//   16 of them past two tiles a CU: 1 x 1 on 230 x 230 3.9 us against 6.7, 10 ->
+//   1000000 fully connected 15 against 43;
+// * and once the layer's own wavefronts fill the GPU and the visits' sources
+//   have to be walked: convergent 5 x 5 on 256 x 256 (1024 tiles) 6.3 us
+//   against 6.8, on 420 x 420 7.4 against 16, 9 x 9 on 420 x 420 17.8 against
+//   28 (on 300 x 300: 15.9 against 15.6).  Fully connected layers need no walk
+//   and keep the tile kernel past 32 visits (20 -> 131072 5.2 us against 6.9,
+//   48 -> 131072 8.3 against 7.1); a sparse one's lists are better read by
+//   whole blocks (64 visits, 2188 tiles: 31 us against 33, 600 visits 319
+//   against 502);
 // * 16 destinations a block while that gives every block a CU of its own
 //   (64 tiles): 784 -> 1024 5.7 us against 11, 4096 -> 4096 24 against 55,
 //   784 -> 8192 (128 tiles) 13.3 against 12.5; not for up to 64 visits,
@@ -55,7 +61,12 @@ template <int TYPE>
 static hipError_t launch_base_type(const sg_conn &c, hipStream_t st) {
     const int tiles = (c.num_dest + 63) / 64;
     const int count = cursor<TYPE>(c, 0).count;
-    if (TYPE != SG_FULLY_CONNECTED && tiles >= (count <= 64 ? 1024 : 2048))
+    const bool lanes =
+        count <= 16 ? tiles > 512
+        : TYPE == SG_FULLY_CONNECTED ? count <= 32 && tiles >= 2048
+        : TYPE == SG_SPARSE ? false
+                            : tiles >= (count <= 64 ? 1024 : 2048);
+    if (lanes)
         launch_lane_type<TYPE>(c, st);
     else if (count > 64 && tiles <= 64)
         launch_tile_type<TYPE, 16, 16>(c, st);

@@ -21,7 +21,10 @@ OUT_BIT, OUT_INT, SUB = 1, 2, 1
 SUBSET, DIV, SPARSE = 1, 4, 5
 
 FULL = [(1, 1), (3, 15), (8, 16), (64, 17), (65, 63), (511, 65), (512, 64),
-        (513, 10), (1100, 33), (100, 64 * 64), (70, 64 * 64 + 1)]
+        (513, 10), (1100, 33), (100, 64 * 64), (70, 64 * 64 + 1),
+        # few visits in many tiles: a lane each, or not
+        (16, 64 * 512), (16, 64 * 512 + 1), (17, 64 * 512 + 1),
+        (32, 64 * 2048), (33, 64 * 2048), (1, 64 * 2048 + 1)]
 
 # rows, columns, field, stride, wrap, offset, shared kernel
 ARBOR = [(1, 1, 3, 1, True, -1, False), (9, 7, 3, 1, False, -1, False),
@@ -30,7 +33,9 @@ ARBOR = [(1, 1, 3, 1, True, -1, False), (9, 7, 3, 1, False, -1, False),
          (256, 256, 3, 1, False, -1, False),
          (257, 256, 3, 1, True, -1, True), (128, 96, 7, 1, True, -3, False),
          (128, 257, 9, 1, False, -4, False), (129, 256, 9, 1, True, -4, False),
-         (256, 256, 9, 1, True, -4, False)]
+         (256, 256, 9, 1, True, -4, False), (256, 256, 6, 1, True, -3, False),
+         (360, 300, 7, 1, False, -3, False), (410, 400, 9, 1, True, -4, True),
+         (192, 180, 4, 1, False, -2, False)]
 
 
 def _serial(x, w):
@@ -230,7 +235,8 @@ def test_subset(size, rect, to, to_rect, out):
 @pytest.mark.gpu
 @pytest.mark.parametrize("out", [OUT_FLOAT, OUT_BIT])
 @pytest.mark.parametrize("n_from,n,K", [(500, 697, 600), (200, 65601, 40),
-                                        (300, 131100, 70)])
+                                        (300, 131100, 70), (90, 66000, 70),
+                                        (90, 33000, 16), (70, 131073, 30)])
 def test_sparse(n_from, n, K, out):
     import torch
     print("sparse", n_from, n, K, out, flush=True)
