@@ -622,33 +622,57 @@ int layer_tiles(int precision, int R) {
 }
 
 // The launch shape of an ensemble that is not given one (sg_ens_set_tile,
-// sg_ens_autotune), from a sweep of every shape, us a step:
+// sg_ens_autotune), by its row tiles and their mean fan-in, from sweeps of
+// every shape; us a step:
 //   8 instances of 128..512 (358 row tiles)    1x8 4.0  2x4 4.0  4x1 5.1
 //   1 of 2048 (256)                            1x8 6.2  2x4 7.3  4x1 13.1
+//   100 of 16 (200)                            1x8 3.3  2x1 3.0  4x1 3.0
 //   64 of 128..1024 (4863)                     2x2 17.4 2x4 18.0 4x1 17.7
 //   64 of 64..256 (1375)                       2x2 4.2  2x4 4.1  4x1 5.4
 //   16 of 1024..2048 (3179)                    2x4 28.7 2x2 30.0 4x1 30.8
 //   256 of 128..4096 (69920)                   2x4 701  2x2 706  4x1 705
+//   1000 of 16..64 (5929)                      2x2 6.3  2x1 4.9  4x1 4.7
+//   1000 of 100 (14000)                        2x2 16.8 2x1 13.1 4x1 13.0
+//   300 of 200 (7800)                          2x2 13.1 2x1 14.9 4x1 14.3
+//   100 of 300..600 (5714)                     2x2 16.9 2x1 16.1 4x1 15.4
+//   3 of 8192 (3072)                           2x4 134  4x4 125  4x1 129
 // Up to two row tiles a CU a step is one wavefront's walk of the fan-in, so
-// eight share it; beyond that blocks of two row tiles start and end more
-// evenly than blocks of four, and long rows are split over four wavefronts.
+// eight share it if it is longer than a load or two; beyond that blocks of
+// two row tiles start and end more evenly than blocks of four, and long rows
+// are split over two or four wavefronts -- but not where so many rows wait
+// that the splits' sums cost more than they shorten.
 // FP32: eight row groups a block (8 instances 4.65 us against 4.80 with
-// four, 1 of 2048 9.0 against 10.9).
+// four, 1 of 2048 9.0 against 10.9); four of short rows (1000 of 100 29.6
+// against 24.8); and where most weights are in rows of a multiple of 2048
+// floats, whose blocks of eight all start on the same memory channels,
+// sixteen (8 of 4096 213 with eight, 181 with four, 171) or, of 2048 itself
+// and past two tiles a CU, four (20 of 2048 143 against 103; 20 of 2000 97
+// against 95).
 void default_shape(sg_ens *e) {
-    long tiles = 0, k = 0;
+    long tiles = 0, k = 0, weights = 0, even = 0, even4 = 0;
     for (const Layer &l : e->layers) {
         tiles += l.tiles;
         k += (long)l.tiles * l.Kp;
+        const long w = (long)l.R * l.Kp;
+        weights += w;
+        if (l.Kp % 2048 == 0) even += w;
+        if (l.Kp % 4096 == 0) even4 += w;
     }
+    const long mean = k / std::max(1L, tiles);
     if (e->precision == SG_ENS_FP32) {
-        e->rt = 8;
         e->ks = 1;
+        if (2 * even4 > weights) e->rt = 16;
+        else if (tiles > 512 && (2 * even > weights || mean <= 128)) e->rt = 4;
+        else e->rt = 8;
     } else if (tiles <= 512) {
-        e->rt = 1;
-        e->ks = 8;
+        e->rt = mean <= 64 ? 2 : 1;
+        e->ks = mean <= 64 ? 1 : 8;
+    } else if (mean <= 64 || (mean < 512 && tiles > (mean < 384 ? 8192 : 4096))) {
+        e->rt = 4;
+        e->ks = 1;
     } else {
-        e->rt = 2;
-        e->ks = k >= 1024 * tiles ? 4 : 2;
+        e->rt = mean >= 8000 ? 4 : 2;
+        e->ks = mean >= 1024 ? 4 : 2;
     }
 }
 

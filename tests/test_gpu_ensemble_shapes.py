@@ -1,10 +1,12 @@
 """The launch shape an ensemble gets by itself, on both sides of its rule's
-lines (512 row tiles, a mean fan-in of 1024), against the shape of one
-wavefront a row tile.
+lines (512, 4096 and 8192 row tiles; a mean fan-in of 64, 384, 512, 1024 and
+8000; FP32 rows of a multiple of 2048), against the shape of one wavefront a
+row tile.
 
 A row's sum is the same products in another grouping: FP32 accumulation over
-up to 1056 terms of size 1/sqrt(1056) differs by far less than 1e-5 of the
-largest state.
+up to 8192 terms of size 1/sqrt(8192) differs by about sqrt(8192) half units
+in the last place of a sum near 1, 3e-6, and less than 1e-5 of the largest
+state.
 """
 
 import numpy as np
@@ -16,8 +18,21 @@ from synaptogenesis_amd.ensemble import RateEnsemble
 SHAPES = [([[40, 4096, 4096]], "bf16", (1, 8)),      # 512 row tiles
           ([[40, 4096, 4097]], "bf16", (2, 4)),      # 513, long rows
           ([[33, 8192, 16], [17, 5, 3]], "bf16", (2, 2)),   # 515, short rows
-          ([[31, 17, 3]], "bf16", (1, 8)),
-          ([[100, 33, 65], [7, 1, 2]], "fp32", (8, 1))]
+          ([[31, 17, 3]], "bf16", (2, 1)),           # fan-ins of one load
+          ([[65, 17, 3]], "bf16", (1, 8)),
+          ([[64, 65, 33]] * 130, "bf16", (2, 2)),    # 1040, mean fan-in 76
+          ([[60, 64, 64]] * 130, "bf16", (4, 1)),    # 1040, 64
+          ([[100, 100, 100]] * 586, "bf16", (4, 1)),     # 8204, 128
+          ([[100, 100, 100]] * 585, "bf16", (2, 2)),     # 8190
+          ([[400, 400, 400]] * 82, "bf16", (4, 1)),      # 4100, 416
+          ([[400, 400, 400]] * 81, "bf16", (2, 2)),      # 4050
+          ([[8192, 8192, 16], [8192, 16, 1]], "bf16", (4, 4)),
+          ([[100, 33, 65], [7, 1, 2]], "fp32", (8, 1)),
+          ([[100, 100, 100]] * 11, "fp32", (4, 1)),      # 550 row groups
+          ([[2048, 2048, 2]], "fp32", (4, 1)),       # 513
+          ([[2048, 2040, 8]], "fp32", (8, 1)),       # 512
+          ([[4096, 100, 4000]], "fp32", (8, 1)),     # even rows in the minority
+          ([[4096, 300, 10]], "fp32", (16, 1))]
 
 
 @pytest.mark.gpu
