@@ -265,11 +265,15 @@ __global__ __launch_bounds__(kNeuronBlock) void gol_neuron_kernel(
     shift_bits(output, size, nid, history, live ? 1u : 0u);
 }
 
-// Up to SG_MAX_FLOAT_BATCH FLOAT layers in one grid, as IzBatch.
+// Up to N FLOAT layers in one grid, as IzBatch.  The arguments are read from
+// the host's memory, so a search for the block's layer is a chain of such
+// reads: a batch of one has none, in a kernel of its own (a relay layer of
+// 100000: 4.4 us a launch with the search, 3.4 without; of 4000000: 6.8, 5.9).
+template <int N>
 struct FloatBatch {
     int n;
-    int first[SG_MAX_FLOAT_BATCH + 1];
-    sg_float_layer l[SG_MAX_FLOAT_BATCH];
+    int first[N + 1];
+    sg_float_layer l[N];
 };
 
 // SG_RATE: re_attribute_kernel (state/impl/rate_encoding_attributes.cpp:
@@ -278,10 +282,12 @@ struct FloatBatch {
 // (state/impl/relay_attributes.cpp:10-18).  A layer is a launch's worth of
 // microseconds by itself (1.3-4 us for 10 to 1024 neurons), so all of a
 // step's layers share one.
+template <int N>
 __global__ __launch_bounds__(kNeuronBlock) void float_neuron_kernel(
-        FloatBatch f) {
+        FloatBatch<N> f) {
     int j = 0;
-    while (j + 1 < f.n && (int)blockIdx.x >= f.first[j + 1]) ++j;
+    if (N > 1)
+        while (j + 1 < f.n && (int)blockIdx.x >= f.first[j + 1]) ++j;
     const sg_float_layer &l = f.l[j];
     const int nid = (blockIdx.x - f.first[j]) * kNeuronBlock + threadIdx.x;
     if (nid >= l.size) return;
@@ -388,16 +394,21 @@ __global__ __launch_bounds__(kNeuronBlock) void copy32_kernel(
 }
 
 // Any n: 16-byte words where both sides allow it, then the tail.  Copy j of
-// the batch has blocks first[j] .. first[j + 1] - 1.
+// the batch has blocks first[j] .. first[j + 1] - 1.  One copy is a batch of
+// its own size, as FloatBatch.
+template <int N>
 struct CopyBatch {
     int n;
-    int first[SG_MAX_COPY_BATCH + 1];
-    sg_copy c[SG_MAX_COPY_BATCH];
+    int first[N + 1];
+    sg_copy c[N];
 };
 
-__global__ __launch_bounds__(kNeuronBlock) void copy_u32_kernel(CopyBatch b) {
+template <int N>
+__global__ __launch_bounds__(kNeuronBlock) void copy_u32_kernel(
+        CopyBatch<N> b) {
     int j = 0;
-    while (j + 1 < b.n && (int)blockIdx.x >= b.first[j + 1]) ++j;
+    if (N > 1)
+        while (j + 1 < b.n && (int)blockIdx.x >= b.first[j + 1]) ++j;
     const uint32_t *src = static_cast<const uint32_t *>(b.c[j].src);
     uint32_t *dst = static_cast<uint32_t *>(b.c[j].dst);
     const long n = b.c[j].n;
@@ -460,7 +471,7 @@ extern "C" int sg_hip_gol_neuron(float *input, uint32_t *output, int size,
 extern "C" int sg_hip_float_neurons(const sg_float_layer *layers, int n,
                                     void *stream) {
     for (int s0 = 0; s0 < n; s0 += SG_MAX_FLOAT_BATCH) {
-        FloatBatch f;
+        FloatBatch<SG_MAX_FLOAT_BATCH> f;
         f.n = 0;
         int blocks = 0;
         for (int j = s0; j < n && j < s0 + SG_MAX_FLOAT_BATCH; ++j) {
@@ -474,8 +485,16 @@ extern "C" int sg_hip_float_neurons(const sg_float_layer *layers, int n,
         }
         if (f.n == 0) continue;
         f.first[f.n] = blocks;
-        hipLaunchKernelGGL(float_neuron_kernel, dim3(blocks),
-                           dim3(kNeuronBlock), 0, (hipStream_t)stream, f);
+        if (f.n == 1) {
+            const FloatBatch<1> one = {1, {0, blocks}, {f.l[0]}};
+            hipLaunchKernelGGL(float_neuron_kernel<1>, dim3(blocks),
+                               dim3(kNeuronBlock), 0, (hipStream_t)stream,
+                               one);
+        } else {
+            hipLaunchKernelGGL(float_neuron_kernel<SG_MAX_FLOAT_BATCH>,
+                               dim3(blocks), dim3(kNeuronBlock), 0,
+                               (hipStream_t)stream, f);
+        }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
@@ -586,7 +605,7 @@ extern "C" int sg_hip_copy32(const void *src, void *dst, long n,
 
 extern "C" int sg_hip_copies_u32(const sg_copy *copies, int n, void *stream) {
     for (int s0 = 0; s0 < n; s0 += SG_MAX_COPY_BATCH) {
-        CopyBatch b;
+        CopyBatch<SG_MAX_COPY_BATCH> b;
         b.n = 0;
         int blocks = 0;
         for (int j = s0; j < n && j < s0 + SG_MAX_COPY_BATCH; ++j) {
@@ -603,8 +622,16 @@ extern "C" int sg_hip_copies_u32(const sg_copy *copies, int n, void *stream) {
         }
         if (b.n == 0) continue;
         b.first[b.n] = blocks;
-        hipLaunchKernelGGL(copy_u32_kernel, dim3(blocks), dim3(kNeuronBlock),
-                           0, (hipStream_t)stream, b);
+        if (b.n == 1) {
+            const CopyBatch<1> one = {1, {0, blocks}, {b.c[0]}};
+            hipLaunchKernelGGL(copy_u32_kernel<1>, dim3(blocks),
+                               dim3(kNeuronBlock), 0, (hipStream_t)stream,
+                               one);
+        } else {
+            hipLaunchKernelGGL(copy_u32_kernel<SG_MAX_COPY_BATCH>,
+                               dim3(blocks), dim3(kNeuronBlock), 0,
+                               (hipStream_t)stream, b);
+        }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
