@@ -22,9 +22,9 @@
 //   backward  checkpoints of at most 16 steps: scan_bwd_fused, the loss
 //             gradient and all of the passes below for every block of
 //             steps in one launch (dW2 summed per batch row), with pack_x
-//             as extra blocks of it; else per block, last first: layer 1's recurrence again from
-//             the block's checkpoint (the currents are kept), recording
-//             v1 and s1, then
+//             as extra blocks of it; else per block, last first: layer
+//             1's recurrence again from the block's checkpoint (the
+//             currents are kept), recording v1 and s1, then
 //             scan2_bwd    one thread per (b, output), steps in reverse:
 //                          d2 = dL/dv2
 //             scan1_bwd    one thread per (b, hidden unit), steps in
@@ -1259,7 +1259,8 @@ __device__ inline float loss_grad_at(const float *__restrict__ counts,
 
 // The whole backward in one launch (checkpoints of at most 16 steps): a
 // block of 256 threads = up to 256 hidden units of one batch row b (ANY:
-// n_hid is not a multiple of 256, so a row's last block is partly idle); it walks the blocks of steps from the last, and per block
+// n_hid is not a multiple of 256, so a row's last block is partly idle); it
+// walks the blocks of steps from the last, and per block
 //  - threads o < O run layer 2's adjoint for (b, o) over the block's steps
 //    exactly as scan2_bwd does, into LDS (every block of the row computes
 //    the same values; the carry stays in a register);
@@ -1352,8 +1353,8 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
             for (int t = 15; t >= 0; --t) {
                 if (t >= a.steps) continue;
                 const float d = (gb - a.reset_theta * dn2) *
-                                act_grad_fast_m<MODE, ANY>(v2[t] - a.theta, a.mode,
-                                                      a.slope) +
+                                act_grad_fast_m<MODE, ANY>(
+                                    v2[t] - a.theta, a.mode, a.slope) +
                                 a.beta * dn2;
                 d2s[t][threadIdx.x] = d;
                 dn2 = d;
@@ -1385,8 +1386,8 @@ __global__ __launch_bounds__(256) void scan_bwd_fused(
                     acc[o] = fmaf(d2s[t][o], sv, acc[o]);
                 }
             const float d = (gs - a.reset_theta * dn) *
-                            act_grad_fast_m<MODE, ANY>(vr[t] - a.theta, a.mode,
-                                                  a.slope) +
+                            act_grad_fast_m<MODE, ANY>(vr[t] - a.theta,
+                                                       a.mode, a.slope) +
                             a.beta * dn;
             if (live) lb[(long)t * BH + i] = d;
             dn = d;
@@ -1580,8 +1581,9 @@ struct Layout {
 // steps fits its LDS table of output adjoints.
 bool fused_backward(const sg_snn_cfg &c) { return c.checkpoint <= 16; }
 
-// dW2 partial-sum slots: one per batch row (fused backward) or per
-// kDw2Rows rows of a block of steps.
+// dW2 partial-sum slots: one per batch row (fused backward: 4 * batch * n_out
+// * n_hid bytes of the workspace, 16 of 162 MB at batch 4096, 25 steps, 64 ->
+// 100 -> 10) or per kDw2Rows rows of a block of steps.
 size_t dw2_slots(const sg_snn_cfg &c) {
     return fused_backward(c)
         ? (size_t)c.batch

@@ -667,7 +667,8 @@ void default_shape(sg_ens *e) {
     } else if (tiles <= 512) {
         e->rt = mean <= 64 ? 2 : 1;
         e->ks = mean <= 64 ? 1 : 8;
-    } else if (mean <= 64 || (mean < 512 && tiles > (mean < 384 ? 8192 : 4096))) {
+    } else if (mean <= 64 ||
+               (mean < 512 && tiles > (mean < 384 ? 8192 : 4096))) {
         e->rt = 4;
         e->ks = 1;
     } else {

@@ -431,9 +431,9 @@ __device__ __forceinline__ uint64_t gol_rule(uint64_t b, uint64_t p,
 // for step s) and, on a bounded board, the cells inside it, by ballot; lane
 // j of the wavefront collects row j's masks.  One wavefront then takes all
 // K steps, lane i = region row i, with the rows above and below from its
-// neighbour lanes (gol_rule).  The count equals the integer sum of the one-weighted
-// bits, which is the float sum of the one-step kernel exactly; cells
-// outside a bounded board hold 0 at every step.  Finally each wavefront
+// neighbour lanes (gol_rule).  The count equals the integer sum of the
+// one-weighted bits, which is the float sum of the one-step kernel exactly;
+// cells outside a bounded board hold 0 at every step.  Finally each wavefront
 // writes its rows' inner words: the staged word shifted by K with the K new
 // bits on top (each lane reads the half of each step's row mask that holds
 // its column), and the last step's count as the input.
@@ -642,7 +642,11 @@ __global__ __launch_bounds__(64) void gol_column_kernel(
     for (int s = 0; s < K; ++s) {
         // gol_life's rule in two-input form.  8 steps a launch, so and with
         // gol_life: 2048 x 2048 17.7 / 16.6 us, 16384 x 16384 429.6 / 431.7
-        // us (bound by HBM there, where boards of this kernel matter most)
+        // us.  There the vector units issue in 70 % of the launch's cycles,
+        // at a clock that falls with the board's density (430 us, 520 on
+        // random words), while 2.9 GB come past the L2 (2.7 times the board:
+        // 64 columns of which 48 are written, off the 128-byte lines) and 1.1
+        // GB go out: neither alone, and fewer instructions gain nothing
         const uint64_t L = gol_from_prev_lane(b);   // the column left
         const uint64_t R = gol_from_next_lane(b);   // the column right
         const uint64_t p = (uint64_t)khi[s] << 32 | klo[s];
@@ -1022,7 +1026,10 @@ extern "C" int sg_hip_gol_steps(const uint32_t *words_in, uint32_t *words_out,
 
 // Steps of a plane launch: sixteen up to four wavefronts a SIMD, where a
 // launch costs its chain rather than its halo (a cell computed four times),
-// eight beyond (2.7 times).
+// eight beyond (2.7 times).  With sixteen and with eight, us a step: 1024 x
+// 1024 0.36 / 0.49, 1536 x 1536 0.63 / 0.67, 2048 x 2048 (4096 wavefronts)
+// 0.68 / 0.75, 2048 x 2112 (4224) 0.94 / 0.83, 4096 x 4096 1.65 / 1.62, 16384 x
+// 16384 34.9 / 28.1.
 static int plane_steps(int rows, int cols) {
     const long waves16 = (long)((cols + 31) / 32) * ((rows + 31) / 32);
     return waves16 <= 4096 ? 16 : 8;

@@ -43,8 +43,8 @@ static void launch_lane_type(const sg_conn &c, hipStream_t st) {
 // Which form of the base activator (all three give the same bits), from one
 // sweep of sizes:
 // * lanes alone where a tile's visits would leave most of a block idle, up to
-//   16 of them past two tiles a CU: 1 x 1 on 230 x 230 3.9 us against 6.7, 10 ->
-//   1000000 fully connected 15 against 43;
+//   16 of them past two tiles a CU: 1 x 1 on 230 x 230 3.9 us against 6.7,
+//   10 -> 1000000 fully connected 15 against 43;
 // * and once the layer's own wavefronts fill the GPU and the visits' sources
 //   have to be walked: convergent 5 x 5 on 256 x 256 (1024 tiles) 6.3 us
 //   against 6.8, on 420 x 420 7.4 against 16, 9 x 9 on 420 x 420 17.8 against

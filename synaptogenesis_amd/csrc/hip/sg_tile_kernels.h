@@ -1,6 +1,6 @@
 // Kernel templates of the tile kernels (base activator and Izhikevich
-// synapse passes), shared by sg_tile.hip (full records) and
-// sg_tile_compact.hip (compact records), which instantiate them.
+// synapse passes), shared by sg_tile.hip (the base activator) and
+// sg_tile_{full,compact}{,_wide}.hip (the passes), which instantiate them.
 #ifndef SG_TILE_KERNELS_H
 #define SG_TILE_KERNELS_H
 
@@ -9,8 +9,8 @@
 // Izhikevich synapse passes (update, activate, fused update+activate).
 //
 // A block owns a tile of 64 destinations.  Its W wavefronts (W = 3, 4 or 16
-// for the Izhikevich passes, chosen per launch) split the tile's synapse list k-wise in
-// chunks of 8 * W (8 visits per wavefront per chunk): every synapse's
+// for the Izhikevich passes, chosen per launch) split the tile's synapse list
+// k-wise in chunks of 8 * W (8 visits per wavefront per chunk): every synapse's
 // independent work -- loads, STDP / short-term plasticity, trace decay,
 // stores -- runs with W wavefronts in flight per tile instead of one.  The
 // only order-dependent part, the FP32 sum over a destination's synapses, is
@@ -512,9 +512,10 @@ static inline int cu_count() {
 // tile per CU: sixteen (the WIDE instantiations), two chunks for a 15 x 15
 // arbor instead of eight and as many memory latencies less: 20 tiles 12 us
 // against 20 with four (260 tiles with sixteen would run a second round:
-// 130 x 128 56 us a step, 128 x 128 45).  Beyond that three or four, whichever lets the whole grid be resident in the fewest rounds of
-// blocks (a grid that overflows the GPU by a fraction runs its last round
-// mostly idle), ties going to four.
+// 130 x 128 56 us a step, 128 x 128 45).  Beyond that three or four, whichever
+// lets the whole grid be resident in the fewest rounds of blocks (a grid that
+// overflows the GPU by a fraction runs its last round mostly idle), ties
+// going to four.
 static inline bool wide_tiles(int tiles) { return tiles <= cu_count(); }
 
 template <class KA, class KB>

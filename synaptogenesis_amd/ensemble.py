@@ -4,8 +4,8 @@ Many independent rate networks of uneven width -- an input layer x0 feeding
 two fully connected rate layers, h1 = layer 1 and h2 = layer 2 -- step
 together: one kernel launch per step over every row of every instance (a
 run of many steps captured once into a HIP graph), or every step of a run
-in one persistent cooperative launch with a grid barrier between steps.  Per step, every layer
-reads the previous step's outputs (the parallel cluster's one-step lag,
+in one persistent cooperative launch with a grid barrier between steps.  Per
+step, every layer reads the previous step's outputs (the parallel cluster's one-step lag,
 engine/cluster/parallel_cluster.cpp:107-131):
 
     h1 <- (1 - leak) h1 + leak f(W1 x0)
