@@ -1829,6 +1829,8 @@ static int backward(const sg_snn_cfg *cfg, const uint16_t *x,
     uint16_t *xp = (uint16_t *)(ws + l.xp);
     if (fused_backward(c)) {
         // the mode and, for 10 outputs, their number fixed at compile time
+        // (784 -> 1000 -> 10, batch 128, 100 steps: 196 us a forward and
+        // backward, 214 with the general form; batch 1024, 50 steps 653, 710)
         typedef void (*BK)(ScanArgs, int, long, const uint16_t *,
                            const float *, const float *, const float *,
                            const float *, const int32_t *, float, float *,

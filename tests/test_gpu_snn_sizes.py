@@ -4,7 +4,7 @@
 The backward scan takes 256 hidden units a block, the products 16-byte rows
 (inputs a multiple of 8, hidden units of 4) in tiles of 112, 128 and 256, the
 output table 16 steps and 16 outputs.  Rate mode, whose gradient is smooth:
-FP32 recurrences of 12 to 32 steps stay within 1e-4 of the largest entry
+FP32 recurrences of up to 32 steps stay within 1e-4 of the largest entry
 (an FP32 rounding, 6e-8, grown by the unit's slope of 12.5 and the steps).
 """
 
